@@ -73,9 +73,7 @@ __global__ __launch_bounds__(kBlock) void frame_load_kernel(FrameLoadParams p) {
     const real_t dx = (x.x - r.x) + static_cast<real_t>(im.x - ri.x) * p.box.L[0];
     const real_t dy = (x.y - r.y) + static_cast<real_t>(im.y - ri.y) * p.box.L[1];
     const real_t dz = (x.z - r.z) + static_cast<real_t>(im.z - ri.z) * p.box.L[2];
-    if (dx * dx + dy * dy + dz * dz > p.threshold_sq) {
-      __hip_atomic_store(&p.ctrl->rebuild, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    raise_flag(dx * dx + dy * dy + dz * dz > p.threshold_sq, &p.ctrl->rebuild);
   }
 }
 

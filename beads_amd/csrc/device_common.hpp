@@ -99,6 +99,18 @@ __device__ __forceinline__ uint32_t wave_increment(uint32_t* counter, uint32_t k
   return result;
 }
 
+// Sets *flag, read by later kernels only, when hit holds in some active lane:
+// one store per wave, into this XCD's L2 (the kernel's end writes it back; all
+// writers store the same word). Stores at agent scope go past the L2 one after
+// another, 37 ns each on one address, which is what a frame_load whose every
+// atom has moved spent its time on (57 of 61 us at 100,000 beads).
+__device__ __forceinline__ void raise_flag(bool hit, uint32_t* flag) {
+  const uint64_t m = __builtin_amdgcn_ballot_w64(hit);
+  if (m != 0 && (threadIdx.x & 63u) == static_cast<uint32_t>(__builtin_ctzll(m))) {
+    __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+}
+
 // 1/x in FP64: the hardware reciprocal (relative error <= 4.6e-8 measured on
 // gfx950) refined by one Newton step (<= 2.3e-15).
 __device__ __forceinline__ double rcp_f64(double x) {
