@@ -74,15 +74,21 @@ __device__ __forceinline__ double team_sum(double v) {
   return v;
 }
 
-// counter[key] += 1 for every active lane of the wave with one atomic per
-// distinct key: the lanes sharing a key add their count through the first of
-// them. Returns the counter's value before this lane's increment (the lanes of
-// a key take consecutive values in lane order).
+// counter[key] += 1 for every active lane of the wave. Up to kSharedKeys
+// distinct keys are served with one atomic each: the lanes sharing a key add
+// their count through the first of them and take consecutive values in lane
+// order. Lanes whose key has not come up by then add for themselves: spatially
+// sorted atoms of a wave lie in a handful of cells, but atoms in a caller's
+// order have a cell each, and one returning atomic after another is a chain of
+// up to 64 memory latencies (cell_scatter of 100,000 shuffled beads). Returns
+// the counter's value before this lane's increment.
+constexpr int kSharedKeys = 6;
+
 __device__ __forceinline__ uint32_t wave_increment(uint32_t* counter, uint32_t key) {
   const uint32_t lane = threadIdx.x & 63u;
   uint64_t pending = __ballot(1);
   uint32_t result = 0;
-  while (pending != 0) {
+  for (int shared = 0; pending != 0 && shared < kSharedKeys; ++shared) {
     const int first = __builtin_ctzll(pending);
     const uint32_t lead = static_cast<uint32_t>(__shfl(static_cast<int>(key), first));
     const uint64_t group = __ballot(key == lead) & pending;
@@ -96,6 +102,7 @@ __device__ __forceinline__ uint32_t wave_increment(uint32_t* counter, uint32_t k
     }
     pending &= ~group;
   }
+  if ((pending >> lane) & 1ull) result = atomicAdd(&counter[key], 1u);
   return result;
 }
 

@@ -27,6 +27,28 @@ def shuffled_lj(n: int, seed: int = 3) -> W.Workload:
     return w.with_(positions=w.positions[order], velocities=w.velocities[order])
 
 
+@pytest.mark.parametrize("n", [1000, 4097, 6400])  # part-filled and whole last waves
+def test_cells_and_lists_of_shuffled_beads(n):
+    w = shuffled_lj(n)
+    plan = O.plan(w)
+    assert plan.path != O.PATH_DIRECT
+    with Engine(w) as e:
+        e.initialize(observables=False)
+        counts, lst = e.neighbors()
+        cells = e.cells(plan.n_cells)
+        st = e.state()
+    ref = O.cell_ids(w, positions=st["positions"])
+    order, ref_counts, offsets = O.stable_cell_order(ref, plan.n_cells, st["positions"])
+    np.testing.assert_array_equal(cells["cell_of"], ref)
+    np.testing.assert_array_equal(cells["cell_count"], ref_counts)
+    np.testing.assert_array_equal(cells["cell_start"], offsets)
+    np.testing.assert_array_equal(cells["cell_atoms"], order)
+    rc, rl, _ = O.neighbor_lists(w, positions=st["positions"], tags=st["tags"], types=st["types"])
+    np.testing.assert_array_equal(counts, rc)
+    for i in range(n):
+        assert np.array_equal(np.sort(lst[:counts[i], i]), np.sort(rl[i, :rc[i]])), i
+
+
 @pytest.mark.parametrize("n", [1000, 4097])
 @pytest.mark.parametrize("moved", ["all", "one"])
 def test_frame_that_moved_rebuilds(n, moved):
