@@ -68,6 +68,12 @@ struct CellGridView {
   int32_t path;  // 0 direct, 1 regular, 2 small dimension
 };
 
+// Sum of the neighbour counts of the current list, in parts a cache line apart
+// (kNeighborParts * kNeighborPartStride words of 8 bytes): the build's
+// workgroups add to them in turn, since one word would serialise them.
+constexpr uint32_t kNeighborParts = 64;
+constexpr uint32_t kNeighborPartStride = 16;
+
 // Device-resident control block. Written only by kernels (and zeroed once at
 // set-up), read back asynchronously by the host.
 struct alignas(256) Ctrl {
@@ -78,7 +84,6 @@ struct alignas(256) Ctrl {
   uint64_t build_count;
   uint64_t dangerous;
   uint64_t reorder_count;
-  uint64_t neighbor_total;  // sum of neighbour counts of the current list
   uint64_t clock;           // steps advanced (counted by the control kernel)
   uint64_t last_sort;       // clock at the last reorder
   double lambda;            // Berendsen factor still to be applied to vel
@@ -192,6 +197,7 @@ struct BuildParams {
   uint32_t* nbr_count;
   uint32_t* nbr;
   Ctrl* ctrl;
+  unsigned long long* neighbor_parts;
   int32_t half;  // keep only partners with a higher slot
   uint32_t stage_cap;  // candidate entries a workgroup may stage in LDS (set by launch_build)
 };

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "device.hpp"
 
@@ -215,6 +216,257 @@ __device__ __forceinline__ CellNeighborhood neighborhood(uint32_t c, const CellG
     h.nz = unique_axis(cz, g.nz, h.zs);
   }
   return h;
+}
+
+// ------------------------------------------------- candidate runs of a build ---
+//
+// A build visits the 27 cells around an atom's cell (fewer on short axes), z
+// outermost, x innermost. Cells adjacent in x are adjacent in the cell-ordered
+// stream, so the three x-cells of a row are one run of the stream, or two where
+// the row wraps around the box (or, with two cells, starts at the upper one).
+
+// Neighbour k (0, 1, 2) along an axis of count cells, in the order of
+// unique_axis, and its image shift code (0: none, 1: +L, 2: -L): with at
+// least 5 cells per axis a candidate in a wrapped neighbour cell lies more
+// than L/2 away (mic adds +L or -L), and in any other neighbour cell less
+// than L/2 away (mic adds 0).
+__device__ inline uint32_t neighbour_cell(uint32_t cc, uint32_t count, int k, uint32_t& code) {
+  code = 0;
+  if (count <= 1) return 0u;
+  if (count == 2) return k == 0 ? (cc == 0 ? 1u : 0u) : cc;
+  if (k == 0) {
+    if (cc == 0) {
+      code = 1;
+      return count - 1;
+    }
+    return cc - 1;
+  }
+  if (k == 2) {
+    if (cc + 1 == count) {
+      code = 2;
+      return 0u;
+    }
+    return cc + 1;
+  }
+  return cc;
+}
+
+__device__ inline real_t shift_of(uint32_t code, real_t L) {
+  return code == 0 ? static_cast<real_t>(0) : (code == 1 ? L : -L);
+}
+
+// Members of cell cc with x-bin below m (cell_xbins; m in 0..kXBins).
+__device__ inline uint32_t members_below(const uint4* xbins, uint32_t cc, int m) {
+  if (m <= 0) return 0u;
+  const uint4 q = xbins[cc];
+  const int f = m - 1;
+  const uint32_t word = (f >> 1) == 0 ? q.x : ((f >> 1) == 1 ? q.y : ((f >> 1) == 2 ? q.z : q.w));
+  return (word >> (16 * (f & 1))) & 0xffffu;
+}
+
+// Rows of x-adjacent cells around an atom (3 along z times 3 along y), and the
+// most runs they make.
+constexpr int kRows = 9;
+constexpr int kMaxRuns = 2 * kRows;
+
+// A run of the stream, [x, y) below 2^28, with the image shift codes of its
+// cells in the top bits: x's in .x, y's and z's in .y.
+constexpr int kRunCodeShift = 28;
+constexpr uint32_t kRunIndexMask = (1u << kRunCodeShift) - 1u;
+
+// The runs of row r (z neighbour r / 3, y neighbour r % 3) of an atom at xi in
+// cell (cx, cy, cz); empty runs are {0, 0}. With 5 or more cells per axis a
+// row whose cells lie at least gy along y and gz along z from the atom holds
+// neighbours only within ext = sqrt(r_s^2 - gy^2 - gz^2) along x, and none when
+// gy^2 + gz^2 > r_s^2: such rows are dropped, and with x-bin tables (xbins,
+// members of a cell ascending in x) the row starts and ends at the bins within
+// ext of the atom, one bin of margin on each side (a bin is an eighth of a
+// cell). The gaps are taken kGapSlack of a cell short, far above the rounding
+// of the cell coordinates, so a skipped member is farther than ext along x, or
+// than the gaps along y and z, by a margin that no rounding of r^2 closes: the
+// accepted candidates and their order are those of the full scan.
+struct RunPair {
+  uint2 a, b;
+};
+__device__ inline RunPair row_run_pair(const CellGridView& g, const BoxView& box, real_t rs2,
+                                       const uint32_t* cell_start, const uint4* xbins, real4 xi,
+                                       uint32_t cx, uint32_t cy, uint32_t cz, uint32_t r) {
+  RunPair out;
+  out.a = out.b = make_uint2(0u, 0u);
+  const int iz = static_cast<int>(r / 3), iy = static_cast<int>(r % 3);
+  if ((iz > 0 && static_cast<uint32_t>(iz) >= g.nz) || (iy > 0 && static_cast<uint32_t>(iy) >= g.ny))
+    return out;
+  uint32_t code_y, code_z;
+  const uint32_t zc = neighbour_cell(cz, g.nz, iz, code_z);
+  const uint32_t rowc = g.nx * (neighbour_cell(cy, g.ny, iy, code_y) + g.ny * zc);
+  // The row's cells [l0, l1] then, where it wraps, [m0, m1]; x shift codes.
+  uint32_t l0, l1, m0 = 1, m1 = 0, code_l = 0, code_m = 0;
+  if (g.nx <= 2) {
+    l0 = 0;
+    l1 = g.nx - 1;
+    if (g.nx == 2 && cx == 0) {
+      l0 = l1 = 1;
+      m0 = m1 = 0;
+    }
+  } else if (cx == 0) {
+    l0 = l1 = g.nx - 1;
+    code_l = 1;
+    m0 = 0;
+    m1 = 1;
+  } else if (cx + 1 == g.nx) {
+    l0 = cx - 1;
+    l1 = cx;
+    m0 = m1 = 0;
+    code_m = 2;
+  } else {
+    l0 = cx - 1;
+    l1 = cx + 1;
+  }
+  uint32_t skip = 0, keep = 0xffffffffu;  // members dropped at the row's start, kept of its last cell
+  uint32_t n_last = 0;
+  const uint32_t last = rowc + (m1 >= m0 ? m1 : l1);
+  if (g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
+    constexpr real_t kGapSlack = static_cast<real_t>(1.0 / 64.0);
+    const real_t fy = (xi.y - box.lo[1]) * g.inv_cell[1] - static_cast<real_t>(cy);
+    const real_t fz = (xi.z - box.lo[2]) * g.inv_cell[2] - static_cast<real_t>(cz);
+    // Gap to the row below (k = 0) and above (k = 2) along one axis.
+    auto gap = [](real_t f, int k, real_t inv_cell) -> real_t {
+      const real_t d = k == 0 ? f - kGapSlack : (static_cast<real_t>(1) - f) - kGapSlack;
+      return k == 1 || d < 0 ? static_cast<real_t>(0) : d / inv_cell;
+    };
+    const real_t gz = gap(fz, iz, g.inv_cell[2]);
+    const real_t gy = gap(fy, iy, g.inv_cell[1]);
+    const real_t ext2 = rs2 - (gy * gy + gz * gz);
+    if (ext2 < 0) return out;
+    if (xbins != nullptr) {
+      const real_t ext = sqrt(ext2);
+      const real_t at = (xi.x - box.lo[0]) * g.inv_cell[0] - static_cast<real_t>(cx);
+      const real_t reach = ext * g.inv_cell[0];
+      // In bins from the start of the left and of the right neighbour cell.
+      const int m_left =
+          static_cast<int>(floor((at - reach + real_t(1)) * static_cast<real_t>(kXBins))) - 1;
+      const int m_right =
+          static_cast<int>(floor((at + reach - real_t(1)) * static_cast<real_t>(kXBins))) + 2;
+      const int ml = m_left < 0 ? 0 : (m_left > kXBins ? kXBins : m_left);
+      const int mr = m_right < 0 ? 0 : (m_right > kXBins ? kXBins : m_right);
+      const uint32_t cl = rowc + l0;
+      const uint32_t n_left = cell_start[cl + 1] - cell_start[cl];
+      n_last = cell_start[last + 1] - cell_start[last];
+      skip = n_left <= kXBinsMaxCount ? members_below(xbins, cl, ml) : 0u;
+      keep = n_last <= kXBinsMaxCount ? members_below(xbins, last, mr) : n_last;
+    }
+  }
+  const uint32_t yz = (code_y | (code_z << 2)) << kRunCodeShift;
+  uint32_t b = cell_start[rowc + l0] + skip, e = cell_start[rowc + l1 + 1];
+  if (m1 < m0 && keep != 0xffffffffu) e -= n_last - keep;
+  if (b < e) out.a = make_uint2(b | (code_l << kRunCodeShift), e | yz);
+  if (m1 >= m0) {
+    b = cell_start[rowc + m0];
+    e = cell_start[rowc + m1 + 1];
+    if (keep != 0xffffffffu) e -= n_last - keep;
+    if (b < e) out.b = make_uint2(b | (code_m << kRunCodeShift), e | yz);
+  }
+  return out;
+}
+
+// A team's runs in visiting order, empty ones left out, into its LDS entry
+// list (kMaxRuns entries); returns how many, the same in every lane. Lane t of
+// TEAM evaluates rows t, t + TEAM, ... Every lane of the team calls it.
+template <int TEAM>
+__device__ inline uint32_t team_runs(const CellGridView& g, const BoxView& box, real_t rs2,
+                                     const uint32_t* cell_start, const uint4* xbins, real4 xi,
+                                     uint32_t c, uint32_t t, uint32_t team_lane0, uint2* runs) {
+  const uint32_t cx = c % g.nx, cyz = c / g.nx, cy = cyz % g.ny, cz = cyz / g.ny;
+  constexpr uint64_t kTeamMask = TEAM >= 64 ? ~0ull : (1ull << TEAM) - 1ull;
+  uint32_t n = 0;
+#pragma unroll 1
+  for (uint32_t r0 = 0; r0 < static_cast<uint32_t>(kRows); r0 += TEAM) {
+    RunPair p;
+    p.a = p.b = make_uint2(0u, 0u);
+    if (r0 + t < static_cast<uint32_t>(kRows)) {
+      p = row_run_pair(g, box, rs2, cell_start, xbins, xi, cx, cy, cz, r0 + t);
+    }
+    const bool has_a = p.a.y != 0, has_b = p.b.y != 0;  // a nonempty run ends past 0
+    const uint64_t ma = (__ballot(has_a) >> team_lane0) & kTeamMask;
+    const uint64_t mb = (__ballot(has_b) >> team_lane0) & kTeamMask;
+    const uint64_t below = (1ull << t) - 1ull;
+    uint32_t at = n + __builtin_popcountll(ma & below) + __builtin_popcountll(mb & below);
+    if (has_a) runs[at++] = p.a;
+    if (has_b) runs[at] = p.b;
+    n += __builtin_popcountll(ma) + __builtin_popcountll(mb);
+  }
+  return n;
+}
+
+// How a build forms a candidate's minimum image.
+constexpr int kShift = 0, kShiftYZ = 1, kGeneric = 2;
+using kShiftMode = std::integral_constant<int, kShift>;
+using kShiftYZMode = std::integral_constant<int, kShiftYZ>;
+using kGenericMode = std::integral_constant<int, kGeneric>;
+
+// One atom's runs scanned by its team of TEAM lanes, TEAM * SLOTS candidates
+// per round, the next round's candidates loaded before this round's are
+// tested (a small system has too few waves to hide a load otherwise). entry(q)
+// is stream entry q = {x, y, z, slot bits}; accept(j, x, mode, shift) the
+// wave's lanes whose candidate is a neighbour; put(slot, j) stores one.
+// Candidates are taken in run order, so neighbours are appended in the order
+// of a one-lane scan. Returns the atom's count, the same in every lane.
+template <int TEAM, int SLOTS, typename Entry, typename Accept, typename Put, typename Mode>
+__device__ __forceinline__ uint32_t scan_runs(const uint2* runs, uint32_t n_runs, uint32_t t,
+                                              uint32_t team_lane0, const BoxView& box, Entry entry,
+                                              Accept accept, Put put, Mode mode) {
+  constexpr uint32_t kRound = TEAM * SLOTS;
+  constexpr uint64_t kTeamMask = TEAM >= 64 ? ~0ull : (1ull << TEAM) - 1ull;
+  const uint64_t below = (1ull << t) - 1ull;
+  uint32_t count = 0;
+  if (n_runs == 0) return count;
+  uint32_t r = 0, k, e;
+  real3 sh;
+  auto open = [&]() {  // run r becomes the current one
+    const uint2 d = runs[r++];
+    k = d.x & kRunIndexMask;
+    e = d.y & kRunIndexMask;
+    const uint32_t yz = d.y >> kRunCodeShift;
+    sh = make_real3(shift_of(d.x >> kRunCodeShift, box.L[0]), shift_of(yz & 3u, box.L[1]),
+                    shift_of(yz >> 2, box.L[2]));
+  };
+  real4 next[SLOTS];
+  auto load = [&]() {  // entries past the run's end repeat its last one
+#pragma unroll
+    for (int u = 0; u < SLOTS; ++u) {
+      const uint32_t q = k + u * TEAM + t;
+      next[u] = entry(q < e ? q : e - 1);
+    }
+  };
+  open();
+  load();
+  for (;;) {
+    real4 x[SLOTS];
+#pragma unroll
+    for (int u = 0; u < SLOTS; ++u) x[u] = next[u];
+    // Slot u of this lane is in the run while u * TEAM < left.
+    const int left = static_cast<int>(e - k) - static_cast<int>(t);
+    const real3 shift = sh;
+    bool more = true;
+    k += kRound;
+    if (k >= e) {
+      more = r < n_runs;
+      if (more) open();
+    }
+    if (more) load();
+#pragma unroll
+    for (int u = 0; u < SLOTS; ++u) {
+      const uint32_t j = id_of(x[u].w);
+      const uint64_t m = __builtin_amdgcn_ballot_w64(u * TEAM < left) & accept(j, x[u], mode, shift);
+      const uint64_t bits = (m >> team_lane0) & kTeamMask;
+      if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+        put(count + static_cast<uint32_t>(__builtin_popcountll(bits & below)), j);
+      }
+      count += static_cast<uint32_t>(__builtin_popcountll(bits));
+    }
+    if (!more) break;
+  }
+  return count;
 }
 
 // LJ pair value in FP64 from the displacement in real_t (exact in binary32

@@ -607,6 +607,8 @@ void Engine::upload_state() {
     pair_acc_.resize(3 * n);
     pair_acc_.zero(stream_);
   }
+  neighbor_parts_.resize(kNeighborParts * kNeighborPartStride);
+  neighbor_parts_.zero(stream_);
   Ctrl c{};
   c.lambda = 1.0;
   ctrl_.upload(&c, 1, stream_);
@@ -707,6 +709,7 @@ void Engine::set_up_params() {
   b.nbr_count = nbr_count_.data();
   b.nbr = nbr_.data();
   b.ctrl = ctrl_.data();
+  b.neighbor_parts = neighbor_parts_.data();
   b.half = half_list_ ? 1 : 0;
 
   BinParams& bp = bin_params_;
@@ -788,7 +791,7 @@ void Engine::set_up_params() {
 // NeighborSystem::rebuild_now (neighbor_system.cpp:107-146) as a predicated
 // launch sequence.
 void Engine::rebuild_sequence(bool forced, uint64_t steps) {
-  launch_control(ctrl_.data(), control_, forced, steps, stream_);
+  launch_control(ctrl_.data(), control_, forced, steps, neighbor_parts_.data(), stream_);
   if (plan_.path != 0) {
     launch_bin(bin_params_, stream_);
     launch_cell_scan(scan_params_, stream_);
@@ -906,6 +909,8 @@ void Engine::check_overflow(const Ctrl& c) {
 }
 
 void Engine::stats(beads_engine_stats_t* out) {
+  std::vector<unsigned long long> parts(neighbor_parts_.size());
+  neighbor_parts_.download(parts.data(), parts.size(), stream_);
   const Ctrl c = fetch_ctrl();
   std::memset(out, 0, sizeof(*out));
   out->step = step_;
@@ -918,7 +923,11 @@ void Engine::stats(beads_engine_stats_t* out) {
   out->ny = plan_.ny;
   out->nz = plan_.nz;
   out->max_neighbors = plan_.max_neighbors;
-  out->mean_neighbors = static_cast<double>(c.neighbor_total) / n_;
+  uint64_t neighbors = 0;
+  for (uint32_t k = 0; k < kNeighborParts; ++k) {
+    neighbors += parts[k * kNeighborPartStride];
+  }
+  out->mean_neighbors = static_cast<double>(neighbors) / n_;
   // Kinetic energy of the velocities as stored (before any pending factor).
   out->ke = ke_from_scale_ ? c.ke : c.ke_pre;
   out->lambda = c.lambda;

@@ -203,6 +203,7 @@ class Engine {
   DeviceBuffer<double> pair_acc_;  // half list: partner-side LJ sums [3 N]
 
   DeviceBuffer<Ctrl> ctrl_;
+  DeviceBuffer<unsigned long long> neighbor_parts_;
   PinnedBuffer<Ctrl> ctrl_host_;
   uint32_t bcap_ = 0, acap_ = 0, dcap_ = 0, ecap_ = 0;
   bool has_topology_ = false;

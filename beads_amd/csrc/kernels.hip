@@ -45,8 +45,11 @@ using namespace dev;
 // cadence counts builds (neighbor_system.cpp:198-202) or, with
 // sort_every_steps, steps: a build sorts when at least that many steps have
 // passed since the last sort (the sort needs the rebuild that follows it).
-__global__ void control_kernel(Ctrl* ctrl, NeighborControl nc, int forced, uint64_t steps) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) {
+__global__ __launch_bounds__(kNeighborParts) void control_kernel(
+    Ctrl* ctrl, NeighborControl nc, int forced, uint64_t steps, unsigned long long* neighbor_parts) {
+  if (forced || ctrl->rebuild) neighbor_parts[threadIdx.x * kNeighborPartStride] = 0;
+  __syncthreads();
+  if (threadIdx.x != 0) {
     return;
   }
   ctrl->clock += steps;
@@ -69,7 +72,6 @@ __global__ void control_kernel(Ctrl* ctrl, NeighborControl nc, int forced, uint6
     ctrl->reorder_count += reorder ? 1u : 0u;
     if (reorder) ctrl->last_sort = ctrl->clock;
     ctrl->checked = 0;
-    ctrl->neighbor_total = 0;
   }
 }
 
@@ -444,78 +446,15 @@ constexpr int kBuildTeam = 4;
 constexpr int kBuildSlots = 4;
 constexpr uint32_t kBuildAtoms = kBlock / kBuildTeam;
 
-// How the build forms a candidate's minimum image (build_kernel's accept).
-constexpr int kShift = 0, kShiftYZ = 1, kGeneric = 2;
-using kShiftMode = std::integral_constant<int, kShift>;
-using kShiftYZMode = std::integral_constant<int, kShiftYZ>;
-using kGenericMode = std::integral_constant<int, kGeneric>;
-
-// Rows of three x-adjacent cells scanned per atom on the rows path (3 along
-// z times 3 along y).
-constexpr int kRows = 9;
-// A row descriptor's end index (below n < 2^28) carries the row's shift codes
-// in its top bits.
-constexpr int kRowCodeShift = 28;
-constexpr uint32_t kRowEndMask = (1u << kRowCodeShift) - 1u;
 // LDS bytes a build workgroup may use to stage the union of its atoms' row
 // runs (more LDS per workgroup costs occupancy).
 constexpr uint32_t kStageBytesMax = 24576;
 
-// Neighbour k (0, 1, 2) along an axis of count cells, in the order of
-// unique_axis, and its image shift code (0: none, 1: +L, 2: -L): with at
-// least 5 cells per axis a candidate in a wrapped neighbour cell lies more
-// than L/2 away (mic adds +L or -L), and in any other neighbour cell less
-// than L/2 away (mic adds 0).
-__device__ inline uint32_t neighbour_cell(uint32_t cc, uint32_t count, int k, uint32_t& code) {
-  code = 0;
-  if (count <= 1) return 0u;
-  if (count == 2) return k == 0 ? (cc == 0 ? 1u : 0u) : cc;
-  if (k == 0) {
-    if (cc == 0) {
-      code = 1;
-      return count - 1;
-    }
-    return cc - 1;
-  }
-  if (k == 2) {
-    if (cc + 1 == count) {
-      code = 2;
-      return 0u;
-    }
-    return cc + 1;
-  }
-  return cc;
-}
-
-__device__ inline real_t shift_of(uint32_t code, real_t L) {
-  return code == 0 ? static_cast<real_t>(0) : (code == 1 ? L : -L);
-}
-
-// Members of cell cc with x-bin below m (cell_xbins; m in 0..kXBins).
-__device__ inline uint32_t members_below(const uint4* xbins, uint32_t cc, int m) {
-  if (m <= 0) return 0u;
-  const uint4 q = xbins[cc];
-  const int f = m - 1;
-  const uint32_t word = (f >> 1) == 0 ? q.x : ((f >> 1) == 1 ? q.y : ((f >> 1) == 2 ? q.z : q.w));
-  return (word >> (16 * (f & 1))) & 0xffffu;
-}
-
 // Rows path: regular grid, at least 5 cells per axis, atom i not in an
-// x-boundary cell. Each row of three x-adjacent cells is one run of the
-// candidate stream, ascending in x (members are in (x, slot) order). A row
-// whose cells lie at least gy along y and gz along z from the atom needs only
-// members within ext = sqrt(r_s^2 - gy^2 - gz^2) along x, and none when
-// gy^2 + gz^2 > r_s^2; the run starts and ends at the x-bins within ext of
-// the atom, one bin of margin on each side (a bin is an eighth of a cell).
-// The gaps are taken kGapSlack of a cell short, far above the rounding of the
-// cell coordinates, so a skipped member is farther than ext along x, or
-// farther than the gaps along y and z, by a margin that no rounding of r^2
-// closes: its r^2 exceeds r_s^2 and the build would reject it. The accepted
-// candidates and their order are those of the full scan. Writes row r (z
-// neighbour r / 3, y neighbour r % 3) as {run begin, run end | (y shift code
-// | z shift code << 2) << kRowCodeShift} for r = t, t + kBuildTeam, ... (the
-// team's lanes share the rows), widens the block's span of row r, [lo[r],
-// hi[r]), to cover a nonempty run, and returns false off the rows path.
+// x-boundary cell, so that each row is one run. Writes row r's run for r = t,
+// t + kBuildTeam, ... (the team's lanes share the rows), widens the block's
+// span of row r, [lo[r], hi[r]), to cover a nonempty run, and returns false
+// off the rows path.
 __device__ inline bool row_runs(const BuildParams& p, uint32_t i, uint32_t t, uint2* rows,
                                 uint32_t* lo_r, uint32_t* hi_r) {
   const CellGridView& g = p.grid;
@@ -523,50 +462,108 @@ __device__ inline bool row_runs(const BuildParams& p, uint32_t i, uint32_t t, ui
   const uint32_t c = p.cell_of[i];
   const uint32_t cx = c % g.nx, cyz = c / g.nx, cy = cyz % g.ny, cz = cyz / g.ny;
   if (cx < 1 || cx + 1 >= g.nx) return false;
-  constexpr real_t kGapSlack = static_cast<real_t>(1.0 / 64.0);
   const real4 xi = p.pos[i];
-  const real_t lo = p.box.lo[0], inv = g.inv_cell[0];
-  const real_t fy = (xi.y - p.box.lo[1]) * g.inv_cell[1] - static_cast<real_t>(cy);
-  const real_t fz = (xi.z - p.box.lo[2]) * g.inv_cell[2] - static_cast<real_t>(cz);
-  // Gap to the row below (k = 0) and above (k = 2) along one axis.
-  auto gap = [](real_t f, int k, real_t inv_cell) -> real_t {
-    const real_t d = k == 0 ? f - kGapSlack : (static_cast<real_t>(1) - f) - kGapSlack;
-    return k == 1 || d < 0 ? static_cast<real_t>(0) : d / inv_cell;
-  };
 #pragma unroll 1
   for (uint32_t r = t; r < static_cast<uint32_t>(kRows); r += kBuildTeam) {
-    const int a = static_cast<int>(r / 3), b = static_cast<int>(r % 3);
-    const real_t gz = gap(fz, a, g.inv_cell[2]);
-    const real_t gy = gap(fy, b, g.inv_cell[1]);
-    const real_t ext2 = p.rs2 - (gy * gy + gz * gz);
-    if (ext2 < 0) {
-      rows[r] = make_uint2(0u, 0u);
-      continue;
-    }
-    const real_t ext = sqrt(ext2);
-    const real_t fl = ((xi.x - ext) - lo) * inv - static_cast<real_t>(cx - 1);
-    const real_t fr = ((xi.x + ext) - lo) * inv - static_cast<real_t>(cx + 1);
-    const int m_left = static_cast<int>(floor(fl * static_cast<real_t>(kXBins))) - 1;
-    const int m_right = static_cast<int>(floor(fr * static_cast<real_t>(kXBins))) + 2;
-    const int ml = m_left < 0 ? 0 : (m_left > kXBins ? kXBins : m_left);
-    const int mr = m_right < 0 ? 0 : (m_right > kXBins ? kXBins : m_right);
-    uint32_t code_y, code_z;
-    const uint32_t zc = neighbour_cell(cz, g.nz, a, code_z);
-    const uint32_t rowc = g.nx * (neighbour_cell(cy, g.ny, b, code_y) + g.ny * zc);
-    const uint32_t cl = rowc + cx - 1, cr = rowc + cx + 1;
-    const uint32_t s_l = p.cell_start[cl], s_m = p.cell_start[cl + 1];
-    const uint32_t s_r = p.cell_start[cr], e_r = p.cell_start[cr + 1];
-    const uint32_t n_l = s_m - s_l, n_r = e_r - s_r;
-    const uint32_t skip_l = n_l <= kXBinsMaxCount ? members_below(p.cell_xbins, cl, ml) : 0u;
-    const uint32_t keep_r = n_r <= kXBinsMaxCount ? members_below(p.cell_xbins, cr, mr) : n_r;
-    const uint32_t b_run = s_l + skip_l, e_run = s_r + keep_r;
-    rows[r] = make_uint2(b_run, e_run | ((code_y | (code_z << 2)) << kRowCodeShift));
-    if (b_run < e_run) {
-      atomicMin(lo_r + r, b_run);
-      atomicMax(hi_r + r, e_run);
+    const uint2 d =
+        row_run_pair(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r).a;
+    rows[r] = d;
+    const uint32_t b = d.x, e = d.y & kRunIndexMask;
+    if (b < e) {
+      atomicMin(lo_r + r, b);
+      atomicMax(hi_r + r, e);
     }
   }
   return true;
+}
+
+// The append rule's test of one atom's candidates: self, distance, exclusions.
+// EXCL: 0 = no exclusions, 4 or 8 = up to that many partners held in
+// registers, -1 = any count read from memory (the spilled ones too).
+template <int EXCL, bool HALF>
+struct BuildAccept {
+  const BuildParams& p;
+  const uint32_t i;
+  const real4 xi;
+  uint32_t ex[EXCL > 0 ? EXCL : 1];
+  uint32_t ne = 0;
+  uint32_t spill_ne = 0, spill_off = 0;  // exclusions past the inline capacity
+
+  __device__ __forceinline__ BuildAccept(const BuildParams& params, uint32_t slot, real4 x)
+      : p(params), i(slot), xi(x) {
+    if (EXCL < 0 && p.spill_index != nullptr) {
+      const uint32_t si = p.spill_index[i];
+      if (si != kNoSpill) {
+        spill_off = p.spill[si].off[3];
+        spill_ne = p.spill[si].cnt[3];
+      }
+    }
+    if (EXCL != 0) {
+      ne = p.topo_count[i] >> 24;
+      if (EXCL > 0) {
+#pragma unroll
+        for (int k = 0; k < EXCL; ++k) {
+          ex[k] = k < static_cast<int>(ne) ? p.excl[static_cast<size_t>(k) * p.n + i] : 0xffffffffu;
+        }
+      }
+    }
+  }
+
+  // sh: the image shift of the candidate's cell, with mic(xi - xj) equal to
+  // (xi - xj) + sh on every axis (cells of a grid with at least 5 cells per
+  // axis). mode: kShift adds sh on every axis, kShiftYZ only on y and z (a run
+  // that does not wrap has no x shift; adding a zero would change nothing but
+  // the sign of a zero difference, which r^2 squares away), kGeneric takes
+  // mic() per candidate.
+  // Returns the wave's lanes that accept their candidate, as a lane mask:
+  // every test is a compare whose ballot is its lane mask, so the tests
+  // combine as scalar ANDs without branches.
+  template <typename Mode>
+  __device__ __forceinline__ uint64_t operator()(uint32_t j, real4 xj, Mode, real3 sh) const {
+    real_t dx, dy, dz;
+    if (Mode::value == kGeneric) {
+      dx = mic(xi.x - xj.x, p.box.L[0], p.box.hL[0]);
+      dy = mic(xi.y - xj.y, p.box.L[1], p.box.hL[1]);
+      dz = mic(xi.z - xj.z, p.box.L[2], p.box.hL[2]);
+    } else {
+      dx = Mode::value == kShift ? (xi.x - xj.x) + sh.x : xi.x - xj.x;
+      dy = (xi.y - xj.y) + sh.y;
+      dz = (xi.z - xj.z) + sh.z;
+    }
+    const real_t r2 = r2_strict(dx, dy, dz);
+    uint64_t m = __builtin_amdgcn_ballot_w64(!(r2 > p.rs2)) &
+                 __builtin_amdgcn_ballot_w64(HALF ? j > i : j != i);
+    if (EXCL > 0) {
+#pragma unroll
+      for (int k = 0; k < EXCL; ++k) {
+        m &= __builtin_amdgcn_ballot_w64(ex[k] != j);
+      }
+    } else if (EXCL < 0) {
+      bool ok = __builtin_amdgcn_inverse_ballot_w64(m);
+      if (ok) {
+        for (uint32_t k = 0; k < ne; ++k) {
+          if (p.excl[static_cast<size_t>(k) * p.n + i] == j) ok = false;
+        }
+        for (uint32_t k = 0; k < spill_ne; ++k) {
+          if (p.spill_excl[spill_off + k] == j) ok = false;
+        }
+      }
+      m = __builtin_amdgcn_ballot_w64(ok);
+    }
+    return m;
+  }
+};
+
+// Stored neighbours and overflow of a workgroup's atoms (stored: this lane's
+// share of the total; over: some atom of this lane found more than fit).
+__device__ __forceinline__ void publish_build(const BuildParams& p, uint32_t stored, bool over,
+                                              double* red_lds) {
+  const double total = block_sum<kBlock>(static_cast<double>(stored), red_lds);
+  if (threadIdx.x == 0) {
+    atomicAdd(&p.neighbor_parts[(blockIdx.x % kNeighborParts) * kNeighborPartStride],
+              static_cast<unsigned long long>(total));
+  }
+  raise_flag(over, &p.ctrl->overflow);
 }
 
 // Full-list build with the append rule of full_neighbor_path_common.cuh:49-94:
@@ -636,10 +633,10 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
       // their row's span).
       for (uint32_t r = t; r < static_cast<uint32_t>(kRows); r += kBuildTeam) {
         const uint2 d = team_rows[r];
-        const uint32_t b_run = d.x, e_run = d.y & kRowEndMask;
+        const uint32_t b_run = d.x, e_run = d.y & kRunIndexMask;
         if (b_run < e_run) {
           const uint32_t shift = stage_off[r] - row_lo[r];
-          team_rows[r] = make_uint2(b_run + shift, ((e_run + shift) & kRowEndMask) | (d.y & ~kRowEndMask));
+          team_rows[r] = make_uint2(b_run + shift, ((e_run + shift) & kRunIndexMask) | (d.y & ~kRunIndexMask));
         }
       }
     }
@@ -648,70 +645,9 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
   if (i < p.n) {  // uniform over a team
     const real4 xi = p.pos[i];
     const uint32_t n = p.n;
-    uint32_t ex[EXCL > 0 ? EXCL : 1];
-    uint32_t ne = 0;
-    uint32_t spill_ne = 0, spill_off = 0;  // exclusions past the inline capacity
-    if (EXCL < 0 && p.spill_index != nullptr) {
-      const uint32_t si = p.spill_index[i];
-      if (si != kNoSpill) {
-        spill_off = p.spill[si].off[3];
-        spill_ne = p.spill[si].cnt[3];
-      }
-    }
-    if (EXCL != 0) {
-      ne = p.topo_count[i] >> 24;
-      if (EXCL > 0) {
-#pragma unroll
-        for (int k = 0; k < EXCL; ++k) {
-          ex[k] = k < static_cast<int>(ne) ? p.excl[static_cast<size_t>(k) * n + i] : 0xffffffffu;
-        }
-      }
-    }
+    const BuildAccept<EXCL, HALF> accept(p, i, xi);
     const real_t L0 = p.box.L[0], L1 = p.box.L[1], L2 = p.box.L[2];
-    const real_t h0 = p.box.hL[0], h1 = p.box.hL[1], h2 = p.box.hL[2];
     const uint32_t maxn = p.max_neighbors;
-    // sh: the image shift of the candidate's cell, with mic(xi - xj) equal to
-    // (xi - xj) + sh on every axis (cells of a regular grid with at least 5
-    // cells per axis). mode: kShift adds sh on every axis, kShiftYZ only on y
-    // and z (a row of x-adjacent cells has no x shift; adding a zero would
-    // change nothing but the sign of a zero difference, which r^2 squares
-    // away), kGeneric takes mic() per candidate.
-    // Returns the wave's lanes that accept their candidate, as a lane mask:
-    // every test is a compare whose ballot is its lane mask, so the tests
-    // combine as scalar ANDs without branches.
-    auto accept = [&](uint32_t j, real4 xj, auto mode, real3 sh) -> uint64_t {
-      real_t dx, dy, dz;
-      if (decltype(mode)::value == kGeneric) {
-        dx = mic(xi.x - xj.x, L0, h0);
-        dy = mic(xi.y - xj.y, L1, h1);
-        dz = mic(xi.z - xj.z, L2, h2);
-      } else {
-        dx = decltype(mode)::value == kShift ? (xi.x - xj.x) + sh.x : xi.x - xj.x;
-        dy = (xi.y - xj.y) + sh.y;
-        dz = (xi.z - xj.z) + sh.z;
-      }
-      const real_t r2 = r2_strict(dx, dy, dz);
-      uint64_t m = __builtin_amdgcn_ballot_w64(!(r2 > p.rs2)) &
-                   __builtin_amdgcn_ballot_w64(HALF ? j > i : j != i);
-      if (EXCL > 0) {
-#pragma unroll
-        for (int k = 0; k < EXCL; ++k) {
-          m &= __builtin_amdgcn_ballot_w64(ex[k] != j);
-        }
-      } else if (EXCL < 0) {
-        bool ok = __builtin_amdgcn_inverse_ballot_w64(m);
-        if (ok) {
-          for (uint32_t k = 0; k < ne; ++k) {
-            if (p.excl[static_cast<size_t>(k) * n + i] == j) ok = false;
-          }
-          for (uint32_t k = 0; k < spill_ne; ++k) {
-            if (p.spill_excl[spill_off + k] == j) ok = false;
-          }
-        }
-        m = __builtin_amdgcn_ballot_w64(ok);
-      }
-      return m;
-    };
     // Candidates [b, e) of a run (b < e) whose entry s is entry(s) = {x, y,
     // z, slot bits}, kBuildTeam * kBuildSlots per round.
     // Atom i's entries of chunk c start at c * chunk_words + row_word.
@@ -778,9 +714,6 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
         return *reinterpret_cast<const real4*>(
             cp_bytes + static_cast<size_t>(k0 * kEntryBytes) + u * kSlotBytes);
       };
-      const int mx = g.nx < 3 ? static_cast<int>(g.nx) : 3;
-      const int my = g.ny < 3 ? static_cast<int>(g.ny) : 3;
-      const int mz = g.nz < 3 ? static_cast<int>(g.nz) : 3;
       // The team's rows in order, one run after another: a team moves to its
       // next row as soon as its run ends, so that the wave's lanes wait only
       // for the team with the most rounds in all, not in each row.
@@ -797,8 +730,8 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
               }
               const uint2 d = team_rows[r++];
               k = d.x;
-              e = d.y & kRowEndMask;
-              const uint32_t code = d.y >> kRowCodeShift;
+              e = d.y & kRunIndexMask;
+              const uint32_t code = d.y >> kRunCodeShift;
               sh = make_real3(0, shift_of(code & 3u, L1), shift_of(code >> 2, L2));
             } while (k >= e);
             if (!more) break;
@@ -807,24 +740,20 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
           k += kBuildTeam * kBuildSlots;
         }
       };
-      auto cells = [&](auto mode) {
+      // Boundary cells and grids of fewer than 5 cells per axis: the rows one
+      // after another, each one run or two.
+      auto rows_in_turn = [&](auto mode) {
 #pragma unroll 1
-        for (int a = 0; a < mz; ++a) {
-          uint32_t code_z;
-          const uint32_t zc = neighbour_cell(cz, g.nz, a, code_z);
-          const real_t sz = shift_of(code_z, L2);
+        for (uint32_t r = 0; r < static_cast<uint32_t>(kRows); ++r) {
+          const RunPair q =
+              row_run_pair(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r);
 #pragma unroll 1
-          for (int b = 0; b < my; ++b) {
-            uint32_t code_y;
-            const uint32_t rowc = g.nx * (neighbour_cell(cy, g.ny, b, code_y) + g.ny * zc);
-            const real_t sy = shift_of(code_y, L1);
-#pragma unroll 1
-            for (int d = 0; d < mx; ++d) {
-              uint32_t code_x;
-              const uint32_t nc = neighbour_cell(cx, g.nx, d, code_x) + rowc;
-              scan_range(p.cell_start[nc], p.cell_start[nc + 1], entry, mode,
-                         make_real3(shift_of(code_x, L0), sy, sz));
-            }
+          for (int part = 0; part < 2; ++part) {
+            const uint2 d = part == 0 ? q.a : q.b;
+            const uint32_t yz = d.y >> kRunCodeShift;
+            scan_range(d.x & kRunIndexMask, d.y & kRunIndexMask, entry, mode,
+                       make_real3(shift_of(d.x >> kRunCodeShift, L0), shift_of(yz & 3u, L1),
+                                  shift_of(yz >> 2, L2)));
           }
         }
       };
@@ -833,9 +762,9 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
       } else if (rows_path) {
         scan_rows(entry);
       } else if (g.path == 1 && g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
-        cells(kShiftMode{});
+        rows_in_turn(kShiftMode{});
       } else {
-        cells(kGenericMode{});
+        rows_in_turn(kGenericMode{});
       }
     }
     if (t == 0) {
@@ -845,15 +774,88 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
     }
   }
   const bool counted = t == 0 && i < p.n;
-  const uint32_t stored = counted ? min(count, p.max_neighbors) : 0u;
-  const double total = block_sum<kBlock>(static_cast<double>(stored), red_lds);
-  if (threadIdx.x == 0) {
-    atomicAdd(reinterpret_cast<unsigned long long*>(&p.ctrl->neighbor_total),
-              static_cast<unsigned long long>(total));
+  publish_build(p, counted ? min(count, p.max_neighbors) : 0u, counted && count > p.max_neighbors,
+                red_lds);
+}
+
+// The build for systems whose atoms make too few waves at kBuildTeam lanes
+// each: kWideTeam lanes per atom, no LDS stage and no workgroup-wide phase.
+// What bounds it is one atom's serial chain (its runs' bounds, then a load per
+// round), so the team covers a row of cells in about one round and the next
+// round's candidates are in flight while this one's are tested.
+constexpr int kWideTeam = 16;
+constexpr int kWideSlots = 4;
+constexpr uint32_t kWideAtoms = kBlock / kWideTeam;
+
+template <int EXCL, bool HALF>
+__global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
+  if (p.ctrl->rebuild == 0) {
+    return;
   }
-  if (counted && count > p.max_neighbors) {
-    atomicOr(&p.ctrl->overflow, 1u);
+  __shared__ double red_lds[4];
+  __shared__ uint2 run_lds[kWideAtoms * kMaxRuns];
+  const uint32_t t = threadIdx.x & (kWideTeam - 1);
+  const uint32_t team_lane0 = (threadIdx.x & 63u) & ~static_cast<uint32_t>(kWideTeam - 1);
+  const uint32_t q = xcd_block(blockIdx.x, gridDim.x) * kWideAtoms + threadIdx.x / kWideTeam;
+  uint2* const runs = run_lds + (threadIdx.x / kWideTeam) * kMaxRuns;
+  const bool direct = p.grid.path == 0;
+  const CellGridView& g = p.grid;
+  real4 xi = make_real4(0, 0, 0, 0);
+  uint32_t i = q, n_runs = 0, count = 0;
+  if (q < p.n) {  // uniform over a team
+    if (direct) {
+      xi = p.pos[q];
+      if (t == 0) runs[0] = make_uint2(0u, p.n);
+      n_runs = 1;
+    } else {
+      xi = p.cell_pos[q];  // the atom's position, .w its slot
+      i = id_of(xi.w);
+      n_runs = team_runs<kWideTeam>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi,
+                                    cell_of_position(xi, p.box, g), t, team_lane0, runs);
+    }
   }
+  __syncthreads();
+  if (q < p.n) {
+    const BuildAccept<EXCL, HALF> accept(p, i, xi);
+    const uint32_t maxn = p.max_neighbors;
+    const uint32_t row_word = i * kNbrChunk;
+    const uint32_t chunk_words = p.n * kNbrChunk;
+    const auto put = [&](uint32_t slot, uint32_t j) {
+      if (slot < maxn) {
+        p.nbr[static_cast<uint64_t>(slot / kNbrChunk) * chunk_words +
+              (row_word | (slot & (kNbrChunk - 1)))] = j;
+      }
+    };
+    if (direct) {
+      const auto entry = [&](uint32_t k) {
+        const real4 x = p.pos[k];
+        return make_real4(x.x, x.y, x.z, real_of_id(k));
+      };
+      count = scan_runs<kWideTeam, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
+                                               put, kGenericMode{});
+    } else {
+      const char* cp_bytes = reinterpret_cast<const char*>(p.cell_pos);
+      const auto entry = [cp_bytes](uint32_t k) {
+        return *reinterpret_cast<const real4*>(cp_bytes +
+                                               k * static_cast<uint32_t>(sizeof(real4)));
+      };
+      if (g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
+        count = scan_runs<kWideTeam, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
+                                                 put, kShiftMode{});
+      } else {
+        count = scan_runs<kWideTeam, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
+                                                 put, kGenericMode{});
+      }
+    }
+    if (t == 0) {
+      p.nbr_count[i] = min(count, maxn);
+      p.ref_pos[i] = xi;
+      p.ref_image[i] = p.image[i];
+    }
+  }
+  const bool counted = t == 0 && q < p.n;
+  publish_build(p, counted ? min(count, p.max_neighbors) : 0u, counted && count > p.max_neighbors,
+                red_lds);
 }
 
 // ------------------------------------------------------------------ force --
@@ -1301,8 +1303,9 @@ __global__ __launch_bounds__(kBlock) void integrate_kernel(IntegrateParams p) {
 }  // namespace
 
 void launch_control(Ctrl* ctrl, NeighborControl control, bool forced, uint64_t steps,
-                    hipStream_t stream) {
-  control_kernel<<<1, 64, 0, stream>>>(ctrl, control, forced ? 1 : 0, steps);
+                    unsigned long long* neighbor_parts, hipStream_t stream) {
+  control_kernel<<<1, kNeighborParts, 0, stream>>>(ctrl, control, forced ? 1 : 0, steps,
+                                                   neighbor_parts);
 }
 
 void launch_bin(const BinParams& p, hipStream_t stream) {
@@ -1332,6 +1335,14 @@ void launch_pack_records(const PackParams& p, hipStream_t stream) {
   pack_records_kernel<<<grid_for(p.n), kBlock, 0, stream>>>(p);
 }
 
+// Atoms up to which the wide build is used. Measured, narrow / wide, us per
+// build (equilibrated systems): bead-spring melt of 8,000 beads 96 / 27, of
+// 27,000 101 / 46, of 64,000 108 / 73, of 100,000 140 / 104, of 216,000
+// 205 / 204, of 512,000 384 / 440; LJ fluid of 500 25 / 10, of 4,000 65 / 17,
+// of 32,000 64 / 38, of 108,000 97 / 83, of 256,000 157 / 171; four-type
+// mixture of 64,000 62 / 56, of 100,000 75 / 76, of 216,000 119 / 139.
+constexpr uint32_t kWideBuildMax = 100000;
+
 void launch_build(const BuildParams& params, hipStream_t stream) {
   const unsigned g = grid_for(params.n, kBuildAtoms);
   // Stage capacity from the mean cell occupancy m: a workgroup's kBuildAtoms
@@ -1349,8 +1360,16 @@ void launch_build(const BuildParams& params, hipStream_t stream) {
   const int ex = p.spill_index != nullptr
                      ? -1
                      : (p.ecap == 0 ? 0 : (p.ecap <= 4 ? 4 : (p.ecap <= 8 ? 8 : -1)));
-#define BEADS_BUILD_CASE(E, H) \
-  if (ex == E && (p.half != 0) == H) build_kernel<E, H><<<g, kBlock, lds, stream>>>(p);
+  const bool wide = p.n <= kWideBuildMax;
+  const unsigned gw = grid_for(params.n, kWideAtoms);
+#define BEADS_BUILD_CASE(E, H)                                          \
+  if (ex == E && (p.half != 0) == H) {                                  \
+    if (wide) {                                                         \
+      build_wide_kernel<E, H><<<gw, kBlock, 0, stream>>>(p);            \
+    } else {                                                            \
+      build_kernel<E, H><<<g, kBlock, lds, stream>>>(p);                \
+    }                                                                   \
+  }
   BEADS_BUILD_CASE(0, false)
   BEADS_BUILD_CASE(4, false)
   BEADS_BUILD_CASE(8, false)
