@@ -796,41 +796,62 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_reorder_commit_kernel(Rep
   });
 }
 
-// Rebuild kernel, one chunk per workgroup: the neighbour lists, with a team
-// of kPhasedBuildTeam adjacent lanes per atom. The candidates are build_atom's
-// in its order (neighbour cells in neighbourhood order, a cell's members in
-// slot order, read from the cell-ordered positions; every atom on the direct
-// path): lane t tests candidates k + u*kPhasedBuildTeam + t of each round and
-// the team appends the accepted ones in candidate order through a ballot, so
+// Rebuild kernel, a quarter of a chunk per workgroup: the neighbour lists, with
+// a team of kPhasedBuildTeam adjacent lanes per atom. The candidates are
+// build_atom's in its order (neighbour cells in neighbourhood order, a cell's
+// members in slot order, read from the cell-ordered positions; every atom on
+// the direct path), as runs of the cell-ordered stream (team_runs), less the
+// rows of cells that lie beyond r_s, whose members build_atom rejects; the team
+// appends the accepted ones in candidate order through a ballot (scan_runs), so
 // the lists are build_atom's. A replica's overflow is the OR over its chunks.
-constexpr int kPhasedBuildTeam = 4;
+// Bound by one atom's chain of runs: a step rebuilds a few replicas, too few
+// atoms to fill the GPU, so an atom takes a quarter wave, whose round covers a
+// row of cells. With four lanes per atom and one run per cell, 27 bounds and
+// twice as many rounds one after another, builds took 99 us per step of 64
+// LJ replicas (about 300,000 beads) and now take 70 (24 melts: 82 and 31).
+constexpr int kPhasedBuildTeam = 16;
 constexpr int kPhasedBuildSlots = 4;
-static_assert(kPhasedBlock == kReplicaChunk * kPhasedBuildTeam, "one chunk per workgroup");
+constexpr uint32_t kPhasedBuildAtoms = kPhasedBlock / kPhasedBuildTeam;
+constexpr uint32_t kBuildParts = kReplicaChunk / kPhasedBuildAtoms;  // workgroups per chunk
 
 // EXCL: 0 no exclusions in the batch; 4 or 8: an atom's excluded partners
 // (at most EXCL) held in registers, unused entries never a slot; -1: read
 // from memory per candidate.
 template <int EXCL>
 __global__ __launch_bounds__(kPhasedBlock) void phased_build_kernel(ReplicaParams P) {
+  __shared__ uint2 run_lds[kPhasedBuildAtoms * kMaxRuns];
   const ReplicaArrays& A = P.arrays;
+  const uint32_t team = threadIdx.x / kPhasedBuildTeam;
   const uint32_t t = threadIdx.x & (kPhasedBuildTeam - 1);
   const uint32_t team_lane0 = (threadIdx.x & 63u) & ~static_cast<uint32_t>(kPhasedBuildTeam - 1);
-  const uint32_t below = (1u << t) - 1u;
-  const uint32_t entries = P.work_count[0];
+  uint2* const runs = run_lds + team * kMaxRuns;
+  const uint32_t entries = P.work_count[0] * kBuildParts;
   for (uint32_t w = blockIdx.x; w < entries; w += gridDim.x) {
-    const ChunkAtoms ca = chunk_atoms(P, wave_uniform(P.work[w]));
+    const ChunkAtoms ca = chunk_atoms(P, wave_uniform(P.work[w / kBuildParts]));
     const ReplicaDesc& d = P.desc[ca.r];
+    const CellGridView& g = d.grid;
     const uint32_t n = d.n;
-    const uint32_t i = ca.a0 + threadIdx.x / kPhasedBuildTeam;
-    uint32_t count = 0;
+    const uint32_t i = ca.a0 + (w % kBuildParts) * kPhasedBuildAtoms + team;
+    const real4* pos = A.pos + d.atom0;
+    uint32_t count = 0, n_runs = 0;
+    real4 xi = make_real4(0, 0, 0, 0);
     if (i < n) {  // uniform over a team
-      const real4* pos = A.pos + d.atom0;
-      const real4* cpos = A.cell_pos + d.atom0;
-      uint32_t* nbr = A.nbr + d.nbr0;
+      xi = pos[i];
+      if (g.path == 0) {
+        if (t == 0) runs[0] = make_uint2(0u, n);
+        n_runs = 1;
+      } else {
+        n_runs = team_runs<kPhasedBuildTeam>(g, d.box, d.rs2, A.cell_start + d.cell0, nullptr, xi,
+                                             A.cell_of[d.atom0 + i], t, team_lane0, runs);
+      }
+    }
+    __syncthreads();
+    if (i < n) {
       const uint32_t maxn = d.max_neighbors;
+      uint32_t* nbr = A.nbr + d.nbr0;
       const real_t L0 = d.box.L[0], L1 = d.box.L[1], L2 = d.box.L[2];
       const real_t h0 = d.box.hL[0], h1 = d.box.hL[1], h2 = d.box.hL[2];
-      const real4 xi = pos[i];
+      const real_t rs2 = d.rs2;
       const uint32_t* excl = A.excl + static_cast<size_t>(P.ecap) * d.atom0;
       const uint32_t ne = EXCL != 0 && d.has_excl ? A.topo_count[d.atom0 + i] >> 24 : 0u;
       uint32_t ex[EXCL > 0 ? EXCL : 1];
@@ -840,63 +861,48 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_build_kernel(ReplicaParam
                     ? excl[static_cast<size_t>(k) * n + i]
                     : 0xffffffffu;
       }
-      const auto excluded = [&](uint32_t j) {
-        bool hit = false;
+      const auto accept = [&](uint32_t j, real4 xj, auto mode, real3 sh) -> uint64_t {
+        real_t dx, dy, dz;
+        if (decltype(mode)::value == kGeneric) {
+          dx = mic(xi.x - xj.x, L0, h0);
+          dy = mic(xi.y - xj.y, L1, h1);
+          dz = mic(xi.z - xj.z, L2, h2);
+        } else {
+          dx = (xi.x - xj.x) + sh.x;
+          dy = (xi.y - xj.y) + sh.y;
+          dz = (xi.z - xj.z) + sh.z;
+        }
+        uint64_t m = __builtin_amdgcn_ballot_w64(!(r2_strict(dx, dy, dz) > rs2)) &
+                     __builtin_amdgcn_ballot_w64(j != i);
         if (EXCL > 0) {
 #pragma unroll
-          for (int k = 0; k < (EXCL > 0 ? EXCL : 1); ++k) hit |= ex[k] == j;
+          for (int k = 0; k < (EXCL > 0 ? EXCL : 1); ++k) {
+            m &= __builtin_amdgcn_ballot_w64(ex[k] != j);
+          }
         } else if (EXCL < 0) {
-          hit = ne != 0 && excluded_partner(excl, n, i, ne, j);
+          m &= __builtin_amdgcn_ballot_w64(!(ne != 0 && excluded_partner(excl, n, i, ne, j)));
         }
-        return hit;
+        return m;
       };
-      // Candidates [b, e) of a run (b < e); entry(k) = {x, y, z, slot bits}.
-      auto scan = [&](uint32_t b, uint32_t e, auto entry) {
-        for (uint32_t k = b; k < e; k += kPhasedBuildTeam * kPhasedBuildSlots) {
-          real4 x[kPhasedBuildSlots];
-#pragma unroll
-          for (int u = 0; u < kPhasedBuildSlots; ++u) {
-            const uint32_t q = k + u * kPhasedBuildTeam + t;
-            x[u] = entry(q < e ? q : e - 1);
-          }
-#pragma unroll
-          for (int u = 0; u < kPhasedBuildSlots; ++u) {
-            const uint32_t j = id_of(x[u].w);
-            const real_t dx = mic(xi.x - x[u].x, L0, h0);
-            const real_t dy = mic(xi.y - x[u].y, L1, h1);
-            const real_t dz = mic(xi.z - x[u].z, L2, h2);
-            const uint64_t m =
-                __builtin_amdgcn_ballot_w64(k + u * kPhasedBuildTeam + t < e) &
-                __builtin_amdgcn_ballot_w64(!(r2_strict(dx, dy, dz) > d.rs2)) &
-                __builtin_amdgcn_ballot_w64(j != i && !excluded(j));
-            const uint32_t bits =
-                static_cast<uint32_t>(m >> team_lane0) & ((1u << kPhasedBuildTeam) - 1u);
-            if (__builtin_amdgcn_inverse_ballot_w64(m)) {
-              const uint32_t slot = count + __builtin_popcount(bits & below);
-              if (slot < maxn) nbr[replica_nbr_index(slot, i, n)] = j;
-            }
-            count += __builtin_popcount(bits);
-          }
-        }
+      const auto put = [&](uint32_t slot, uint32_t j) {
+        if (slot < maxn) nbr[replica_nbr_index(slot, i, n)] = j;
       };
-      if (d.grid.path == 0) {
-        scan(0u, n, [pos](uint32_t k) {
-          const real4 q = pos[k];
-          return make_real4(q.x, q.y, q.z, real_of_id(k));
-        });
+      if (g.path == 0) {
+        const auto entry = [pos](uint32_t k) {
+          const real4 x = pos[k];
+          return make_real4(x.x, x.y, x.z, real_of_id(k));
+        };
+        count = scan_runs<kPhasedBuildTeam, kPhasedBuildSlots>(runs, n_runs, t, team_lane0, d.box,
+                                                               entry, accept, put, kGenericMode{});
       } else {
-        const uint32_t* start = A.cell_start + d.cell0;
+        const real4* cpos = A.cell_pos + d.atom0;
         const auto entry = [cpos](uint32_t k) { return cpos[k]; };
-        const CellNeighborhood h = neighborhood(A.cell_of[d.atom0 + i], d.grid);
-        for (int a = 0; a < h.nz; ++a) {
-          for (int b = 0; b < h.ny; ++b) {
-            const uint32_t row = d.grid.nx * (h.ys[b] + d.grid.ny * h.zs[a]);
-            for (int c = 0; c < h.nx; ++c) {
-              const uint32_t cell = h.xs[c] + row;
-              const uint32_t b0 = start[cell], e0 = start[cell + 1];
-              if (b0 < e0) scan(b0, e0, entry);
-            }
-          }
+        if (g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
+          count = scan_runs<kPhasedBuildTeam, kPhasedBuildSlots>(
+              runs, n_runs, t, team_lane0, d.box, entry, accept, put, kShiftMode{});
+        } else {
+          count = scan_runs<kPhasedBuildTeam, kPhasedBuildSlots>(
+              runs, n_runs, t, team_lane0, d.box, entry, accept, put, kGenericMode{});
         }
       }
       if (t == 0) {
@@ -909,6 +915,7 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_build_kernel(ReplicaParam
         (threadIdx.x & 63u) == 0) {
       atomicOr(&P.state[ca.r].overflow, 1u);
     }
+    __syncthreads();  // the runs are read before the next part's are written
   }
 }
 
@@ -1052,14 +1059,16 @@ void launch_phased_step(const ReplicaParams& p, PhasedShape shape, bool initial,
   phased_rank_kernel<<<work, kPhasedBlock, 0, stream>>>(p);
   phased_reorder_gather_kernel<<<work, kPhasedBlock, 0, stream>>>(p);
   phased_reorder_commit_kernel<<<work, kPhasedBlock, 0, stream>>>(p);
+  const unsigned work_build =
+      std::min<unsigned>(kBuildParts * kWorkBlocks, p.total_chunks * kBuildParts);
   if (p.ecap == 0) {
-    phased_build_kernel<0><<<work, kPhasedBlock, 0, stream>>>(p);
+    phased_build_kernel<0><<<work_build, kPhasedBlock, 0, stream>>>(p);
   } else if (p.ecap <= 4) {
-    phased_build_kernel<4><<<work, kPhasedBlock, 0, stream>>>(p);
+    phased_build_kernel<4><<<work_build, kPhasedBlock, 0, stream>>>(p);
   } else if (p.ecap <= 8) {
-    phased_build_kernel<8><<<work, kPhasedBlock, 0, stream>>>(p);
+    phased_build_kernel<8><<<work_build, kPhasedBlock, 0, stream>>>(p);
   } else {
-    phased_build_kernel<-1><<<work, kPhasedBlock, 0, stream>>>(p);
+    phased_build_kernel<-1><<<work_build, kPhasedBlock, 0, stream>>>(p);
   }
   const int kick = initial ? 0 : 1;
   const bool obs = observables || initial;
