@@ -74,13 +74,17 @@ struct CellGridView {
 constexpr uint32_t kNeighborParts = 64;
 constexpr uint32_t kNeighborPartStride = 16;
 
+// Ctrl::overflow when a wait between a rebuild's workgroups passed its bound.
+constexpr uint32_t kRebuildStalled = 2;
+
 // Device-resident control block. Written only by kernels (and zeroed once at
 // set-up), read back asynchronously by the host.
 struct alignas(256) Ctrl {
   uint32_t rebuild;         // a rebuild is due in this step
   uint32_t reorder;         // the rebuild also sorts particles into cell order
+  uint32_t joined;          // workgroups that joined this step's rebuild (rebuild_kernel)
   uint32_t checked;         // a scheduled check ran since the last build
-  uint32_t overflow;        // a neighbour list overflowed
+  uint32_t overflow;        // 1: a neighbour list overflowed; kRebuildStalled
   uint64_t build_count;
   uint64_t dangerous;
   uint64_t reorder_count;
@@ -239,7 +243,6 @@ struct ReorderParams {
   uint32_t* cell_atoms;
   real4* cell_pos;
   uint32_t* new_of_old;
-  Ctrl* ctrl;
 };
 
 }  // namespace beads_amd

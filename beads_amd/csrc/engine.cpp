@@ -609,6 +609,9 @@ void Engine::upload_state() {
   }
   neighbor_parts_.resize(kNeighborParts * kNeighborPartStride);
   neighbor_parts_.zero(stream_);
+  sync_lines_.resize(2 * kRebuildMaxBlocks * kSyncLine);
+  sync_lines_.zero(stream_);
+  tile_sums_.resize(kRebuildMaxBlocks);
   Ctrl c{};
   c.lambda = 1.0;
   ctrl_.upload(&c, 1, stream_);
@@ -712,15 +715,6 @@ void Engine::set_up_params() {
   b.neighbor_parts = neighbor_parts_.data();
   b.half = half_list_ ? 1 : 0;
 
-  BinParams& bp = bin_params_;
-  bp.n = n_;
-  bp.pos = pos_.data();
-  bp.box = box_;
-  bp.grid = grid;
-  bp.cell_of = cell_of_.data();
-  bp.cell_count = cell_count_.data();
-  bp.ctrl = ctrl_.data();
-
   CellScanParams& sp = scan_params_;
   sp.n = n_;
   sp.n_cells = plan_.n_cells;
@@ -734,7 +728,12 @@ void Engine::set_up_params() {
   sp.cell_xbins = cell_xbins_.data();
   sp.box = box_;
   sp.grid = grid;
-  sp.ctrl = ctrl_.data();
+
+  RebuildParams& rb = rebuild_params_;
+  rb.ctrl = ctrl_.data();
+  rb.neighbor_parts = neighbor_parts_.data();
+  rb.sync_lines = sync_lines_.data();
+  rb.tile_sums = tile_sums_.data();
 
   ReorderParams& r = reorder_params_;
   r.n = n_;
@@ -774,7 +773,6 @@ void Engine::set_up_params() {
   r.cell_atoms = cell_atoms_.data();
   r.cell_pos = cell_pos_.data();
   r.new_of_old = new_of_old_.data();
-  r.ctrl = ctrl_.data();
 
   ScaleParams& sc = scale_params_;
   sc.n = n_;
@@ -791,13 +789,13 @@ void Engine::set_up_params() {
 // NeighborSystem::rebuild_now (neighbor_system.cpp:107-146) as a predicated
 // launch sequence.
 void Engine::rebuild_sequence(bool forced, uint64_t steps) {
-  launch_control(ctrl_.data(), control_, forced, steps, neighbor_parts_.data(), stream_);
   if (plan_.path != 0) {
-    launch_bin(bin_params_, stream_);
-    launch_cell_scan(scan_params_, stream_);
-    launch_cell_scatter(scan_params_, stream_);
-    launch_cell_sort(scan_params_, stream_);
-    launch_reorder(reorder_params_, stream_);
+    rebuild_params_.control = control_;
+    rebuild_params_.forced = forced ? 1 : 0;
+    rebuild_params_.steps = steps;
+    launch_rebuild(scan_params_, reorder_params_, rebuild_params_, stream_);
+  } else {
+    launch_control(ctrl_.data(), control_, forced, steps, neighbor_parts_.data(), stream_);
   }
   launch_build(build_params_, stream_);
 }
@@ -896,6 +894,8 @@ Ctrl Engine::fetch_ctrl() {
 }
 
 void Engine::check_overflow(const Ctrl& c) {
+  require(c.overflow != kRebuildStalled, "the neighbor rebuild's workgroups lost each other.",
+          BEADS_E_DEVICE);
   if (c.overflow != 0) {
     std::ostringstream m;
     m << "NeighborList overflow"
@@ -1186,7 +1186,8 @@ void Engine::frame_load(const real_t* positions_dev, bool reuse_list, bool async
   frame_loaded_ = false;
   load_frame(positions_dev, reuse_list);
   // The force pass normally clears the rebuild flags; no force pass runs here.
-  BEADS_HIP(hipMemsetAsync(ctrl_.data(), 0, 2 * sizeof(uint32_t), stream_));
+  static_assert(offsetof(Ctrl, joined) == 2 * sizeof(uint32_t), "rebuild, reorder, joined lead Ctrl");
+  BEADS_HIP(hipMemsetAsync(ctrl_.data(), 0, 3 * sizeof(uint32_t), stream_));
   BEADS_HIP(hipGetLastError());
   if (!async) check_overflow(fetch_ctrl());
   frame_loaded_ = true;

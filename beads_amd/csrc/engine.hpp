@@ -204,6 +204,8 @@ class Engine {
 
   DeviceBuffer<Ctrl> ctrl_;
   DeviceBuffer<unsigned long long> neighbor_parts_;
+  DeviceBuffer<uint64_t> sync_lines_;  // rebuild_kernel's meeting points
+  DeviceBuffer<uint32_t> tile_sums_;
   PinnedBuffer<Ctrl> ctrl_host_;
   uint32_t bcap_ = 0, acap_ = 0, dcap_ = 0, ecap_ = 0;
   bool has_topology_ = false;
@@ -224,7 +226,7 @@ class Engine {
   ForceParams force_params_{};
   IntegrateParams integrate_params_{};
   BuildParams build_params_{};
-  BinParams bin_params_{};
+  RebuildParams rebuild_params_{};
   CellScanParams scan_params_{};
   ReorderParams reorder_params_{};
   ScaleParams scale_params_{};

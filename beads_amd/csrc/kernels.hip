@@ -45,29 +45,28 @@ using namespace dev;
 // cadence counts builds (neighbor_system.cpp:198-202) or, with
 // sort_every_steps, steps: a build sorts when at least that many steps have
 // passed since the last sort (the sort needs the rebuild that follows it).
-__global__ __launch_bounds__(kNeighborParts) void control_kernel(
-    Ctrl* ctrl, NeighborControl nc, int forced, uint64_t steps, unsigned long long* neighbor_parts) {
-  if (forced || ctrl->rebuild) neighbor_parts[threadIdx.x * kNeighborPartStride] = 0;
-  __syncthreads();
-  if (threadIdx.x != 0) {
-    return;
-  }
+__device__ __forceinline__ bool reorder_due(const Ctrl* ctrl, const NeighborControl& nc,
+                                            uint64_t steps) {
+  const bool due = nc.sort_every_steps != 0
+                       ? ctrl->clock + steps - ctrl->last_sort >= nc.sort_every_steps
+                       : ((ctrl->build_count + 1) % nc.sort_every) == 0;
+  return nc.path != 0 && due;
+}
+
+// One thread: the counters of a step, with the decisions taken from them.
+__device__ __forceinline__ void update_control(Ctrl* ctrl, const NeighborControl& nc, bool forced,
+                                               bool rebuild, bool reorder, uint64_t steps) {
   ctrl->clock += steps;
-  if (forced) {
-    ctrl->rebuild = 1;
-  } else {
+  if (!forced) {
     const bool first = ctrl->checked == 0;
     ctrl->checked = 1;
-    if (ctrl->rebuild && nc.check_every > 1 && first) {
+    if (rebuild && nc.check_every > 1 && first) {
       ctrl->dangerous += 1;
     }
   }
-  if (ctrl->rebuild) {
+  if (rebuild) {
+    ctrl->rebuild = 1;
     ctrl->build_count += 1;
-    const bool due = nc.sort_every_steps != 0
-                         ? ctrl->clock - ctrl->last_sort >= nc.sort_every_steps
-                         : (ctrl->build_count % nc.sort_every) == 0;
-    const bool reorder = nc.path != 0 && due;
     ctrl->reorder = reorder ? 1u : 0u;
     ctrl->reorder_count += reorder ? 1u : 0u;
     if (reorder) ctrl->last_sort = ctrl->clock;
@@ -75,110 +74,236 @@ __global__ __launch_bounds__(kNeighborParts) void control_kernel(
   }
 }
 
-// cell_list_build.cu:135-166: binary32 cell index and atomic counts.
-__global__ __launch_bounds__(kBlock) void bin_kernel(BinParams p) {
-  if (p.ctrl->rebuild == 0) {
-    return;
+// Direct path: the bookkeeping alone, no cells to bin.
+__global__ __launch_bounds__(kNeighborParts) void control_kernel(
+    Ctrl* ctrl, NeighborControl nc, int forced, uint64_t steps, unsigned long long* neighbor_parts) {
+  const bool rebuild = forced || ctrl->rebuild;
+  if (rebuild) neighbor_parts[threadIdx.x * kNeighborPartStride] = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    update_control(ctrl, nc, forced != 0, rebuild, rebuild && reorder_due(ctrl, nc, steps), steps);
   }
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= p.n) {
-    return;
+}
+
+// ----------------------------------------------------- one-launch rebuild --
+//
+// Binning, scan, scatter, in-cell sort and reorder are phases of one kernel:
+// as kernels of their own, with the bookkeeping, they were seven launches a
+// step, most of which find no rebuild due (about 2 us each inside a step
+// graph). The phases are separated by barriers over the grid's workgroups.
+// 100 steps of a 48,000-bead melt 4.98 -> 4.06 ms. A rebuild itself takes
+// 26 us there, 85 us for the 1,000,000-bead melt (95 us as separate kernels)
+// and 305 us with a reorder, most of it memory; of a small one (25 us at 4,000
+// beads) most is the barriers, 4 us each.
+//
+// Which workgroups take part is settled at run time, so that no wait depends
+// on how many of them the GPU holds at once: a workgroup that starts joins by
+// taking a rank; rank 0 closes the list when all have joined, or kJoinTicks
+// after its own start, and a workgroup that starts later leaves at once. The
+// members are all running when the list closes and wait only for each other,
+// so every wait ends. Work is divided by rank over the members there are.
+//
+// Each member has a cache line of its own to arrive on and one to be released
+// on: polls and stores of 256 workgroups on one word would serialise (33 ns
+// each past the L2).
+constexpr int kRebuildBlock = 1024;
+constexpr uint32_t kRebuildWaves = kRebuildBlock / 64;
+constexpr uint32_t kJoinClosed = 0x80000000u;
+constexpr uint32_t kRankBits = 9;  // ranks and counts up to kRebuildMaxBlocks
+static_assert(kRebuildMaxBlocks < (1u << kRankBits) && kRebuildMaxBlocks <= kRebuildBlock,
+              "rank 0 polls one member per thread");
+// wall_clock64 ticks (100 MHz): how long rank 0 waits for the grid to start,
+// and the bound on any other wait, which only a fault can reach.
+constexpr long long kJoinTicks = 3000;
+constexpr long long kWaitTicks = 400000000;
+
+struct Members {
+  uint64_t* lines;  // [member][2 * kSyncLine]: arrival word, release word a line later
+  uint32_t rank, count;
+  uint64_t epoch;   // unique to this rebuild and barrier, advanced by each barrier
+};
+
+template <typename T>
+__device__ __forceinline__ T agent_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void agent_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits until *word holds the epoch above its kRankBits; false past the bound.
+__device__ __forceinline__ bool await_epoch(const uint64_t* word, uint64_t epoch) {
+  const long long start = wall_clock64();
+  while ((agent_load(word) >> kRankBits) != epoch) {
+    if (wall_clock64() - start > kWaitTicks) return false;
+    __builtin_amdgcn_s_sleep(1);
   }
+  return true;
+}
+
+// Joins the rebuild's members. Returns false (in every thread) where the
+// workgroup has nothing to do. epoch0 is above 0, which the lines start with.
+__device__ __forceinline__ bool join_members(Ctrl* ctrl, uint64_t* lines, uint64_t epoch0,
+                                             Members& m) {
+  __shared__ uint32_t rank_lds, count_lds;
+  if (threadIdx.x == 0) {
+    const uint32_t v = __hip_atomic_fetch_add(&ctrl->joined, 1u, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+    rank_lds = v;
+    count_lds = 0;
+    if (v == 0) {
+      const long long start = wall_clock64();
+      while (agent_load(&ctrl->joined) < gridDim.x && wall_clock64() - start < kJoinTicks) {
+        __builtin_amdgcn_s_sleep(1);
+      }
+      count_lds = __hip_atomic_fetch_or(&ctrl->joined, kJoinClosed, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  __syncthreads();
+  const uint32_t rank = rank_lds;
+  if (rank & kJoinClosed) return false;
+  m.lines = lines;
+  m.rank = rank;
+  m.epoch = epoch0;
+  if (rank == 0) {
+    const uint32_t count = count_lds;
+    if (threadIdx.x > 0 && threadIdx.x < count) {
+      agent_store(lines + (2 * threadIdx.x + 1) * kSyncLine, (epoch0 << kRankBits) | count);
+    }
+  } else if (threadIdx.x == 0) {
+    const uint64_t* const release = lines + (2 * rank + 1) * kSyncLine;
+    if (await_epoch(release, epoch0)) {
+      count_lds = static_cast<uint32_t>(agent_load(release)) & ((1u << kRankBits) - 1u);
+    } else {
+      agent_store(&ctrl->overflow, kRebuildStalled);
+    }
+  }
+  __syncthreads();
+  m.count = count_lds;
+  return m.count != 0;
+}
+
+// Barrier over the members. What they stored at agent scope (agent_store,
+// atomics) before it is seen by agent_load and atomics after it: such accesses
+// go past the L2, which another XCD does not see, so all the barrier has to do
+// is wait for them. FULL also hands over ordinary stores, by writing back and
+// emptying the L2, 2 us a barrier and more where it holds much: only the
+// reorder moves enough data to want it. Returns false (in every thread) past
+// the bound on a wait.
+template <bool FULL>
+__device__ __forceinline__ bool member_barrier(Ctrl* ctrl, Members& m) {
+  __shared__ int ok_lds;
+  m.epoch += 1;
+  if (threadIdx.x == 0) ok_lds = 1;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are acknowledged
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (FULL) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (m.rank != 0) agent_store(m.lines + 2 * m.rank * kSyncLine, m.epoch << kRankBits);
+  }
+  if (m.rank == 0) {
+    if (threadIdx.x > 0 && threadIdx.x < m.count &&
+        !await_epoch(m.lines + 2 * threadIdx.x * kSyncLine, m.epoch)) {
+      ok_lds = 0;
+    }
+    __syncthreads();
+    if (threadIdx.x > 0 && threadIdx.x < m.count && ok_lds) {
+      agent_store(m.lines + (2 * threadIdx.x + 1) * kSyncLine, m.epoch << kRankBits);
+    }
+  } else if (threadIdx.x == 0 &&
+             !await_epoch(m.lines + (2 * m.rank + 1) * kSyncLine, m.epoch)) {
+    ok_lds = 0;
+  }
+  __syncthreads();
+  const bool ok = ok_lds != 0;
+  if (!ok && threadIdx.x == 0) agent_store(&ctrl->overflow, kRebuildStalled);
+  // One wave's acquire empties the caches the workgroup reads through.
+  if (FULL && threadIdx.x < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  __syncthreads();
+  return ok;
+}
+
+// Exclusive scan of a value over the workgroup's threads; total gets the sum.
+__device__ __forceinline__ uint32_t block_exclusive(uint32_t v, uint32_t* lds, uint32_t& total) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  uint32_t incl = v;
+#pragma unroll
+  for (uint32_t off = 1; off < 64; off <<= 1) {
+    const uint32_t u = __shfl_up(incl, off, 64);
+    incl += lane >= off ? u : 0u;
+  }
+  __syncthreads();
+  if (lane == 63) lds[wave] = incl;
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kRebuildWaves; ++w) {
+    const uint32_t x = lds[w];
+    before += w < wave ? x : 0u;
+    total += x;
+  }
+  return before + incl - v;
+}
+
+// cell_list_build.cu:135-166: cell index in the storage precision and atomic
+// counts, one atomic per distinct cell of the wave.
+__device__ __forceinline__ void bin_atom(const CellScanParams& p, uint32_t i) {
   const uint32_t c = cell_of_position(p.pos[i], p.box, p.grid);
   p.cell_of[i] = c;
-  wave_increment(p.cell_count, c);  // one atomic per distinct cell of the wave
+  wave_increment(p.cell_count, c);
 }
 
-// One workgroup: exclusive scan of cell counts into cell_start[0..n_cells],
-// copy to the scatter cursor and clear the counts for the next rebuild. The
-// counts pass through LDS in tiles of kScanTile cells: coalesced loads (all
-// of a thread's loads in flight), a scan of kScanPer consecutive cells per
-// thread, a shuffle scan of the thread sums within each wave and the wave
-// totals added from LDS (four barriers per tile), coalesced stores. Rows
-// are padded by one word per kScanPer so a thread's row starts in its own
-// bank.
-constexpr int kScanBlock = 1024;
-constexpr uint32_t kScanPer = 8;
-constexpr uint32_t kScanTile = kScanBlock * kScanPer;
+// Cells up to which a member sums the counts before its own tile by itself
+// (at most 64 KB from the L2) instead of a further barrier.
+constexpr uint32_t kOwnPrefixCells = 16384;
 
-__device__ __forceinline__ uint32_t scan_slot(uint32_t k) { return k + k / kScanPer; }
-
-__global__ __launch_bounds__(kScanBlock) void cell_scan_kernel(CellScanParams p) {
-  if (p.ctrl->rebuild == 0) {
-    return;
-  }
-  constexpr uint32_t kWaves = kScanBlock / 64;
-  __shared__ uint32_t tile[kScanTile + kScanBlock];
-  __shared__ uint32_t wave_total[kWaves];
+// Exclusive scan of the cell counts into cell_start[0..n_cells], copied to the
+// scatter cursor; clears the counts for the next rebuild. Each member scans
+// its own tile of consecutive cells.
+__device__ __forceinline__ bool scan_cells(const CellScanParams& p, Ctrl* ctrl, Members& m,
+                                           uint32_t* tile_sums) {
+  __shared__ uint32_t lds[kRebuildWaves];
   const uint32_t t = threadIdx.x;
-  const uint32_t lane = t & 63u, wave = t >> 6;
-  uint32_t carry = 0;
-  for (uint32_t base = 0; base < p.n_cells; base += kScanTile) {
-    const uint32_t len = min(kScanTile, p.n_cells - base);
-#pragma unroll
-    for (uint32_t m = 0; m < kScanPer; ++m) {
-      const uint32_t k = m * kScanBlock + t;
-      tile[scan_slot(k)] = k < len ? p.cell_count[base + k] : 0u;
-    }
-    __syncthreads();
-    uint32_t local = 0;
-#pragma unroll
-    for (uint32_t m = 0; m < kScanPer; ++m) {
-      local += tile[scan_slot(t * kScanPer + m)];
-    }
-    uint32_t incl = local;  // inclusive scan of the thread sums within the wave
-#pragma unroll
-    for (uint32_t off = 1; off < 64; off <<= 1) {
-      const uint32_t v = __shfl_up(incl, off, 64);
-      incl += lane >= off ? v : 0u;
-    }
-    if (lane == 63) wave_total[wave] = incl;
-    __syncthreads();
-    uint32_t before = 0, tile_total = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < kWaves; ++w) {
-      const uint32_t v = wave_total[w];
-      before += w < wave ? v : 0u;
-      tile_total += v;
-    }
-    uint32_t run = carry + before + incl - local;
-#pragma unroll
-    for (uint32_t m = 0; m < kScanPer; ++m) {
-      const uint32_t s = scan_slot(t * kScanPer + m);
-      const uint32_t cnt = tile[s];
-      tile[s] = run;
-      run += cnt;
-    }
-    carry += tile_total;
-    __syncthreads();
-#pragma unroll
-    for (uint32_t m = 0; m < kScanPer; ++m) {
-      const uint32_t k = m * kScanBlock + t;
-      if (k < len) {
-        const uint32_t start = tile[scan_slot(k)];
-        p.cell_start[base + k] = start;
-        p.cell_cursor[base + k] = start;
-        p.cell_count[base + k] = 0;
-      }
-    }
-    __syncthreads();
+  const uint32_t per = (p.n_cells + m.count - 1) / m.count;
+  const uint32_t begin = min(p.n_cells, m.rank * per), end = min(p.n_cells, begin + per);
+  uint32_t mine = 0, carry = 0;
+  if (p.n_cells <= kOwnPrefixCells) {
+    for (uint32_t c = t; c < begin; c += kRebuildBlock) mine += agent_load(p.cell_count + c);
+    block_exclusive(mine, lds, carry);
+  } else {
+    uint32_t total;
+    for (uint32_t c = begin + t; c < end; c += kRebuildBlock) mine += agent_load(p.cell_count + c);
+    block_exclusive(mine, lds, total);
+    if (t == 0) agent_store(tile_sums + m.rank, total);
+    if (!member_barrier<false>(ctrl, m)) return false;
+    block_exclusive(t < m.rank ? agent_load(tile_sums + t) : 0u, lds, carry);
   }
-  if (t == 0) {
-    p.cell_start[p.n_cells] = carry;
+  // Other members may still sum this tile's counts: they are cleared past the
+  // next barrier.
+  for (uint32_t base = begin; base < end; base += kRebuildBlock) {
+    const uint32_t c = base + t;
+    const uint32_t cnt = c < end ? agent_load(p.cell_count + c) : 0u;
+    uint32_t total;
+    const uint32_t start = carry + block_exclusive(cnt, lds, total);
+    if (c < end) {
+      agent_store(p.cell_start + c, start);
+      agent_store(p.cell_cursor + c, start);
+    }
+    carry += total;
   }
+  if (end == p.n_cells && t == 0) agent_store(p.cell_start + p.n_cells, carry);
+  if (!member_barrier<false>(ctrl, m)) return false;
+  for (uint32_t c = begin + t; c < end; c += kRebuildBlock) p.cell_count[c] = 0;
+  return true;
 }
 
-__global__ __launch_bounds__(kBlock) void cell_scatter_kernel(CellScanParams p) {
-  if (p.ctrl->rebuild == 0) {
-    return;
-  }
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= p.n) {
-    return;
-  }
-  // One atomic per distinct cell of the wave; cell_sort orders the members.
+// Counting-sort scatter of an atom into its cell; sort_cell orders the members.
+__device__ __forceinline__ void scatter_atom(const CellScanParams& p, uint32_t i) {
   const uint32_t slot = wave_increment(p.cell_cursor, p.cell_of[i]);
-  p.cell_atoms[slot] = i;
+  agent_store(p.cell_atoms + slot, i);
 }
 
 // Order each cell's members by (x, slot): with the counting sort this is a
@@ -193,8 +318,6 @@ __global__ __launch_bounds__(kBlock) void cell_scatter_kernel(CellScanParams p) 
 // is insertion-sorted by lane 0. When no reorder follows, the kernel also
 // writes the members' positions in cell order with the slot in .w (the
 // build's candidate stream); after a reorder, reorder_commit writes them.
-constexpr uint32_t kSortCellsPerBlock = kBlock / 64;
-
 __device__ __forceinline__ real4 cell_entry(real4 x, uint32_t slot) {
   return make_real4(x.x, x.y, x.z, real_of_id(slot));
 }
@@ -227,69 +350,61 @@ __device__ __forceinline__ bool before_in_cell(real_t xa, uint32_t sa, real_t xb
   return xa < xb || (xa == xb && sa < sb);
 }
 
-__global__ __launch_bounds__(kBlock) void cell_sort_kernel(CellScanParams p) {
-  if (p.ctrl->rebuild == 0) {
-    return;
-  }
+// One wave orders cell c; stream: also write the candidate stream.
+__device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, bool stream) {
   const uint32_t lane = threadIdx.x & 63u;
-  const bool stream = p.ctrl->reorder == 0;
   const real_t lo = p.box.lo[0], inv = p.grid.inv_cell[0];
-  // A capped grid loops over the cells, so the launch stays small when the
-  // rebuild flag makes it exit at once.
-  for (uint32_t c = blockIdx.x * kSortCellsPerBlock + threadIdx.x / 64; c < p.n_cells;
-       c += gridDim.x * kSortCellsPerBlock) {  // uniform over the wave
-    const uint32_t b = p.cell_start[c], e = p.cell_start[c + 1];
-    const uint32_t cnt = e - b;
-    const uint32_t cx = c % p.grid.nx;
-    uint32_t* a = p.cell_atoms;
-    if (cnt <= 64) {
-      const uint32_t v = lane < cnt ? a[b + lane] : 0xffffffffu;
-      const real4 xv4 = lane < cnt ? p.pos[v] : make_real4(0, 0, 0, 0);
-      const real_t xv = xv4.x;
-      uint32_t rank = 0;
-      for (uint32_t m = 0; m < cnt; ++m) {
-        const uint32_t w = static_cast<uint32_t>(
-            __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(m)));
-        const real_t xw = read_lane(xv, static_cast<int>(m));
-        rank += before_in_cell(xw, w, xv, v) ? 1u : 0u;
-      }
-      if (lane < cnt) {
-        a[b + rank] = v;
-        if (stream) p.cell_pos[b + rank] = cell_entry(xv4, v);
-      }
-      const int bin = lane < cnt ? x_bin(xv, lo, inv, cx) : kXBins;
-      uint32_t pre[kXBins];
+  const uint32_t b = agent_load(p.cell_start + c), e = agent_load(p.cell_start + c + 1);
+  const uint32_t cnt = e - b;
+  const uint32_t cx = c % p.grid.nx;
+  uint32_t* a = p.cell_atoms;
+  if (cnt <= 64) {
+    const uint32_t v = lane < cnt ? agent_load(a + b + lane) : 0xffffffffu;
+    const real4 xv4 = lane < cnt ? p.pos[v] : make_real4(0, 0, 0, 0);
+    const real_t xv = xv4.x;
+    uint32_t rank = 0;
+    for (uint32_t m = 0; m < cnt; ++m) {
+      const uint32_t w = static_cast<uint32_t>(
+          __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(m)));
+      const real_t xw = read_lane(xv, static_cast<int>(m));
+      rank += before_in_cell(xw, w, xv, v) ? 1u : 0u;
+    }
+    if (lane < cnt) {
+      a[b + rank] = v;
+      if (stream) p.cell_pos[b + rank] = cell_entry(xv4, v);
+    }
+    const int bin = lane < cnt ? x_bin(xv, lo, inv, cx) : kXBins;
+    uint32_t pre[kXBins];
 #pragma unroll
-      for (int m = 1; m <= kXBins; ++m) {
-        pre[m - 1] = static_cast<uint32_t>(__builtin_popcountll(__ballot(bin < m)));
+    for (int m = 1; m <= kXBins; ++m) {
+      pre[m - 1] = static_cast<uint32_t>(__builtin_popcountll(__ballot(bin < m)));
+    }
+    if (lane == 0) {
+      p.cell_xbins[c] = make_uint4(pre[0] | (pre[1] << 16), pre[2] | (pre[3] << 16),
+                                   pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
+    }
+  } else if (lane == 0) {
+    for (uint32_t k = b + 1; k < e; ++k) {
+      const uint32_t v = a[k];
+      const real_t xv = p.pos[v].x;
+      uint32_t m = k;
+      while (m > b && before_in_cell(xv, v, p.pos[a[m - 1]].x, a[m - 1])) {
+        a[m] = a[m - 1];
+        --m;
       }
-      if (lane == 0) {
-        p.cell_xbins[c] = make_uint4(pre[0] | (pre[1] << 16), pre[2] | (pre[3] << 16),
-                                     pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
-      }
-    } else if (lane == 0) {
-      for (uint32_t k = b + 1; k < e; ++k) {
-        const uint32_t v = a[k];
-        const real_t xv = p.pos[v].x;
-        uint32_t m = k;
-        while (m > b && before_in_cell(xv, v, p.pos[a[m - 1]].x, a[m - 1])) {
-          a[m] = a[m - 1];
-          --m;
-        }
-        a[m] = v;
-      }
-      uint32_t pre[kXBins] = {};
-      for (uint32_t k = b; k < e; ++k) {
-        const uint32_t v = a[k];
-        const real4 xv4 = p.pos[v];
-        if (stream) p.cell_pos[k] = cell_entry(xv4, v);
-        const int bin = x_bin(xv4.x, lo, inv, cx);
-        for (int m = bin + 1; m <= kXBins; ++m) ++pre[m - 1];
-      }
-      if (cnt <= kXBinsMaxCount) {
-        p.cell_xbins[c] = make_uint4(pre[0] | (pre[1] << 16), pre[2] | (pre[3] << 16),
-                                     pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
-      }
+      a[m] = v;
+    }
+    uint32_t pre[kXBins] = {};
+    for (uint32_t k = b; k < e; ++k) {
+      const uint32_t v = a[k];
+      const real4 xv4 = p.pos[v];
+      if (stream) p.cell_pos[k] = cell_entry(xv4, v);
+      const int bin = x_bin(xv4.x, lo, inv, cx);
+      for (int m = bin + 1; m <= kXBins; ++m) ++pre[m - 1];
+    }
+    if (cnt <= kXBinsMaxCount) {
+      p.cell_xbins[c] = make_uint4(pre[0] | (pre[1] << 16), pre[2] | (pre[3] << 16),
+                                   pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
     }
   }
 }
@@ -344,14 +459,7 @@ __global__ __launch_bounds__(kBlock) void pack_records_kernel(PackParams p) {
 
 // cell_list_build.cu:183-219: gather every per-atom array into cell order
 // (new slot s takes old slot cell_atoms[s]) and record the inverse map.
-__global__ __launch_bounds__(kBlock) void reorder_gather_kernel(ReorderParams p) {
-  if (p.ctrl->rebuild == 0 || p.ctrl->reorder == 0) {
-    return;
-  }
-  const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= p.n) {
-    return;
-  }
+__device__ __forceinline__ void gather_atom(const ReorderParams& p, uint32_t s) {
   const uint32_t o = p.cell_atoms[s];
   p.new_of_old[o] = s;
   p.s_pos[s] = p.pos[o];
@@ -370,14 +478,7 @@ __global__ __launch_bounds__(kBlock) void reorder_gather_kernel(ReorderParams p)
 }
 
 // Copy back and translate partner slots through the inverse permutation.
-__global__ __launch_bounds__(kBlock) void reorder_commit_kernel(ReorderParams p) {
-  if (p.ctrl->rebuild == 0 || p.ctrl->reorder == 0) {
-    return;
-  }
-  const uint32_t s = blockIdx.x * kBlock + threadIdx.x;
-  if (s >= p.n) {
-    return;
-  }
+__device__ __forceinline__ void commit_atom(const ReorderParams& p, uint32_t s) {
   p.pos[s] = p.s_pos[s];
   p.vel[s] = p.s_vel[s];
   p.image[s] = p.s_image[s];
@@ -440,6 +541,47 @@ __global__ __launch_bounds__(kBlock) void reorder_commit_kernel(ReorderParams p)
       }
     }
   }
+}
+
+// Phases 1 to 6 of a rebuild for the atoms and cells of this member; see the
+// section's head. The build that follows is a launch of its own: it wants far
+// more workgroups than wait at a barrier.
+__global__ __launch_bounds__(kRebuildBlock) void rebuild_kernel(CellScanParams cp, ReorderParams rp,
+                                                                RebuildParams p) {
+  Ctrl* const ctrl = p.ctrl;
+  const bool forced = p.forced != 0;
+  const bool rebuild = forced || ctrl->rebuild != 0;
+  if (!rebuild) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      update_control(ctrl, p.control, false, false, false, p.steps);
+    }
+    return;
+  }
+  const bool reorder = reorder_due(ctrl, p.control, p.steps);
+  Members m;
+  if (!join_members(ctrl, p.sync_lines, (ctrl->build_count + 1) * 8u, m)) return;
+  const uint32_t n = cp.n;
+  const uint32_t first = m.rank * kRebuildBlock + threadIdx.x;
+  const uint32_t stride = m.count * kRebuildBlock;
+  for (uint64_t i = first; i < n; i += stride) bin_atom(cp, static_cast<uint32_t>(i));
+  if (!member_barrier<false>(ctrl, m)) return;
+  // Every member has read the counters that its decisions come from.
+  if (m.rank == 0) {
+    if (threadIdx.x < kNeighborParts) p.neighbor_parts[threadIdx.x * kNeighborPartStride] = 0;
+    if (threadIdx.x == 0) update_control(ctrl, p.control, forced, true, reorder, p.steps);
+  }
+  if (!scan_cells(cp, ctrl, m, p.tile_sums)) return;
+  for (uint64_t i = first; i < n; i += stride) scatter_atom(cp, static_cast<uint32_t>(i));
+  if (!member_barrier<false>(ctrl, m)) return;
+  for (uint32_t c = m.rank * kRebuildWaves + threadIdx.x / 64; c < cp.n_cells;
+       c += m.count * kRebuildWaves) {  // uniform over the wave
+    sort_cell(cp, c, !reorder);
+  }
+  if (!reorder) return;
+  if (!member_barrier<true>(ctrl, m)) return;
+  for (uint64_t s = first; s < n; s += stride) gather_atom(rp, static_cast<uint32_t>(s));
+  if (!member_barrier<true>(ctrl, m)) return;
+  for (uint64_t s = first; s < n; s += stride) commit_atom(rp, static_cast<uint32_t>(s));
 }
 
 constexpr int kBuildTeam = 4;
@@ -1146,6 +1288,7 @@ __global__ __launch_bounds__(kReduceBlock) void step_reduce_kernel(ForceParams p
   if (threadIdx.x == 0) {
     p.ctrl->rebuild = 0;
     p.ctrl->reorder = 0;
+    p.ctrl->joined = 0;
     if (HALF) {
       p.ctrl->half_pair[0] = 0.0;
       p.ctrl->half_pair[1] = 0.0;
@@ -1308,27 +1451,15 @@ void launch_control(Ctrl* ctrl, NeighborControl control, bool forced, uint64_t s
                                                    neighbor_parts);
 }
 
-void launch_bin(const BinParams& p, hipStream_t stream) {
-  bin_kernel<<<grid_for(p.n), kBlock, 0, stream>>>(p);
-}
-
-void launch_cell_scan(const CellScanParams& p, hipStream_t stream) {
-  cell_scan_kernel<<<1, kScanBlock, 0, stream>>>(p);
-}
-
-void launch_cell_scatter(const CellScanParams& p, hipStream_t stream) {
-  cell_scatter_kernel<<<grid_for(p.n), kBlock, 0, stream>>>(p);
-}
-
-void launch_cell_sort(const CellScanParams& p, hipStream_t stream) {
-  constexpr unsigned kMaxSortBlocks = 4096;
-  const unsigned g = grid_for(p.n_cells, kSortCellsPerBlock);
-  cell_sort_kernel<<<g < kMaxSortBlocks ? g : kMaxSortBlocks, kBlock, 0, stream>>>(p);
-}
-
-void launch_reorder(const ReorderParams& p, hipStream_t stream) {
-  reorder_gather_kernel<<<grid_for(p.n), kBlock, 0, stream>>>(p);
-  reorder_commit_kernel<<<grid_for(p.n), kBlock, 0, stream>>>(p);
+void launch_rebuild(const CellScanParams& cells, const ReorderParams& reorder,
+                    const RebuildParams& p, hipStream_t stream) {
+  // More workgroups than the atoms fill shorten the per-cell phase; four times
+  // as many as kRebuildBlock asks for took 39 instead of 43 us per rebuild at
+  // 100,000 atoms, 26 instead of 30 at 48,000 and 25 instead of 27 at 4,000.
+  // Half the cap costs 134 instead of 85 us at 1,000,000.
+  const unsigned g = grid_for(cells.n, kRebuildBlock / 4);
+  rebuild_kernel<<<g < kRebuildMaxBlocks ? g : kRebuildMaxBlocks, kRebuildBlock, 0, stream>>>(
+      cells, reorder, p);
 }
 
 void launch_pack_records(const PackParams& p, hipStream_t stream) {

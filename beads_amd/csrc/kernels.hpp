@@ -9,21 +9,10 @@ namespace beads_amd {
 
 constexpr int kBlock = 256;
 
-struct BinParams {
-  uint32_t n;
-  const real4* pos;
-  BoxView box;
-  CellGridView grid;
-  uint32_t* cell_of;
-  uint32_t* cell_count;
-  Ctrl* ctrl;
-  NeighborControl control;
-};
-
 struct CellScanParams {
   uint32_t n;
   uint32_t n_cells;
-  const uint32_t* cell_of;
+  uint32_t* cell_of;
   uint32_t* cell_count;
   uint32_t* cell_start;
   uint32_t* cell_cursor;
@@ -33,7 +22,19 @@ struct CellScanParams {
   uint4* cell_xbins; // per cell: x-bin prefix counts of its x-sorted members
   BoxView box;
   CellGridView grid;
+};
+
+// The rebuild kernel's bookkeeping and the memory its workgroups meet in.
+constexpr uint32_t kRebuildMaxBlocks = 256;
+constexpr uint32_t kSyncLine = 16;  // 8-byte words of a member's arrival or release line
+struct RebuildParams {
   Ctrl* ctrl;
+  NeighborControl control;
+  int32_t forced;
+  uint64_t steps;                      // steps advanced since the previous launch
+  unsigned long long* neighbor_parts;  // cleared for the build
+  uint64_t* sync_lines;                // [kRebuildMaxBlocks][2 * kSyncLine], zero at set-up
+  uint32_t* tile_sums;                 // [kRebuildMaxBlocks]
 };
 
 struct ScaleParams {
@@ -63,14 +64,13 @@ constexpr uint32_t kCandidatePad = 16;
 
 // Neighbour-rebuild sequence; every kernel is predicated on ctrl->rebuild so
 // the host never waits for the displacement check.
-// steps: steps advanced since the previous control launch (0 at set-up).
+// The bookkeeping alone (direct path). steps: steps advanced since the
+// previous launch (0 at set-up).
 void launch_control(Ctrl* ctrl, NeighborControl control, bool forced, uint64_t steps,
                     unsigned long long* neighbor_parts, hipStream_t stream);
-void launch_bin(const BinParams& p, hipStream_t stream);
-void launch_cell_scan(const CellScanParams& p, hipStream_t stream);
-void launch_cell_scatter(const CellScanParams& p, hipStream_t stream);
-void launch_cell_sort(const CellScanParams& p, hipStream_t stream);
-void launch_reorder(const ReorderParams& p, hipStream_t stream);
+// Binning, scan, scatter, sort and (when due) reorder: one launch.
+void launch_rebuild(const CellScanParams& cells, const ReorderParams& reorder,
+                    const RebuildParams& p, hipStream_t stream);
 void launch_build(const BuildParams& p, hipStream_t stream);
 
 // Trajectory records in file order (slot order), one `words`-word record per

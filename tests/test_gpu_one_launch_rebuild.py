@@ -1,0 +1,63 @@
+"""The rebuild kernel's phases (binning, scan, scatter, sort, reorder in one
+launch) where its work splits differently: part-filled and single workgroups,
+more cells than a workgroup sums the prefix of by itself, cells of more than a
+wave's members.
+
+Every step rebuilds and reorders (zero skin, sort at every build), so each phase
+hands over to the next many times before the final cells, in-cell order and
+neighbour sets are held bit for bit to the oracle's at the final positions.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle as O
+from beads_amd import workloads as W
+from beads_amd.capi import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+def _final_state(w, steps):
+    with Engine(w) as e:
+        e.initialize(observables=False)
+        e.advance(steps)
+        plan = O.plan(w)
+        st, cells, stats = e.state(), e.cells(plan.n_cells), e.stats()
+        counts, lst = e.neighbors()
+    assert stats.overflow == 0
+    assert stats.build_count == steps + 1 and stats.reorder_count >= steps
+    ref = O.cell_ids(w, positions=st["positions"])
+    order, ref_counts, offsets = O.stable_cell_order(ref, plan.n_cells, st["positions"])
+    np.testing.assert_array_equal(cells["cell_count"], ref_counts)
+    np.testing.assert_array_equal(cells["cell_start"], offsets)
+    np.testing.assert_array_equal(cells["cell_atoms"], order)
+    assert sorted(st["tags"]) == list(range(1, w.n + 1))
+    rc, rl, ovf = O.neighbor_lists(w, positions=st["positions"], tags=st["tags"], types=st["types"])
+    assert not ovf
+    np.testing.assert_array_equal(counts, rc)
+    for i in range(0, w.n, max(1, w.n // 3000)):
+        assert np.array_equal(np.sort(lst[:counts[i], i]), np.sort(rl[i, :rc[i]])), i
+
+
+def _every_step(w):
+    return w.with_(cutoff_buffer=0.0, sort_every_rebuild=1)
+
+
+@pytest.mark.parametrize("n", [500, 1023, 1024, 1025, 5000])
+def test_part_filled_workgroups(n):
+    _final_state(_every_step(W.lj_box(n, 0.8, 1.0, seed=n)), 40)
+
+
+def test_more_cells_than_one_prefix():
+    w = _every_step(W.lj_box(20000, 0.05, 1.0, seed=2))
+    assert O.plan(w).n_cells > 16384
+    _final_state(w, 24)
+
+
+def test_cells_of_more_than_a_wave():
+    w = _every_step(W.lj_box(6000, 0.8, 1.0, seed=4, cutoff=5.0)).with_(max_neighbors=768)
+    assert w.n / O.plan(w).n_cells > 64
+    _final_state(w, 10)
