@@ -418,41 +418,14 @@ void Batch::replica_stats(uint32_t r, beads_engine_stats_t* out) {
 void Batch::read_state(uint32_t r, const beads_state_out_t& o) {
   require(r < count_, "replica index out of range.", BEADS_E_INDEX);
   const ReplicaDesc& d = desc_host_[position_of_[r]];
-  const size_t n = d.n, a0 = d.atom0;
-  std::vector<real4> pos(n), vel(n), force(n);
-  std::vector<int4> img(n);
-  BEADS_HIP(hipMemcpyAsync(pos.data(), pos_.data() + a0, n * sizeof(real4), hipMemcpyDeviceToHost, stream_));
-  BEADS_HIP(hipMemcpyAsync(vel.data(), vel_.data() + a0, n * sizeof(real4), hipMemcpyDeviceToHost, stream_));
-  BEADS_HIP(hipMemcpyAsync(force.data(), force_.data() + a0, n * sizeof(real4), hipMemcpyDeviceToHost, stream_));
-  BEADS_HIP(hipMemcpyAsync(img.data(), image_.data() + a0, n * sizeof(int4), hipMemcpyDeviceToHost, stream_));
-  if (o.tags) {
-    BEADS_HIP(hipMemcpyAsync(o.tags, tag_.data() + a0, n * sizeof(uint32_t), hipMemcpyDeviceToHost, stream_));
-  }
-  synchronize();
-  for (size_t i = 0; i < n; ++i) {
-    if (o.positions) {
-      o.positions[3 * i] = pos[i].x;
-      o.positions[3 * i + 1] = pos[i].y;
-      o.positions[3 * i + 2] = pos[i].z;
-    }
-    if (o.types) o.types[i] = static_cast<int32_t>(id_of(pos[i].w)) + 1;
-    if (o.velocities) {
-      o.velocities[3 * i] = vel[i].x;
-      o.velocities[3 * i + 1] = vel[i].y;
-      o.velocities[3 * i + 2] = vel[i].z;
-    }
-    if (o.masses) o.masses[i] = vel[i].w;
-    if (o.forces) {
-      o.forces[3 * i] = force[i].x;
-      o.forces[3 * i + 1] = force[i].y;
-      o.forces[3 * i + 2] = force[i].z;
-    }
-    if (o.images) {
-      o.images[3 * i] = img[i].x;
-      o.images[3 * i + 1] = img[i].y;
-      o.images[3 * i + 2] = img[i].z;
-    }
-  }
+  StateSource src;
+  src.n = d.n;
+  src.pos = pos_.data() + d.atom0;
+  src.vel = vel_.data() + d.atom0;
+  src.force = force_.data() + d.atom0;
+  src.image = image_.data() + d.atom0;
+  src.tag = tag_.data() + d.atom0;
+  state_reader_.read(src, o, stream_);
 }
 
 }  // namespace beads_amd

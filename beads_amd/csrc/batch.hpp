@@ -5,6 +5,7 @@
 
 #include "common.hpp"
 #include "replicas.hpp"
+#include "state_reader.hpp"
 
 namespace beads_amd {
 
@@ -56,6 +57,7 @@ class Batch {
   std::vector<uint4> init_angle_, init_dih_;
   std::vector<CachedGraph> graphs_;
   hipStream_t stream_ = nullptr;
+  StateReader state_reader_;
 
   DeviceBuffer<ReplicaDesc> desc_;
   DeviceBuffer<ReplicaState> state_;

@@ -943,40 +943,16 @@ void Engine::stats(beads_engine_stats_t* out) {
 }
 
 void Engine::read_state(const beads_state_out_t& o) {
-  const size_t n = n_;
-  std::vector<real4> pos(n), vel(n), force(n);
-  std::vector<int4> img(n);
-  pos_.download(pos.data(), n, stream_);
-  vel_.download(vel.data(), n, stream_);
-  force_.download(force.data(), n, stream_);
-  image_.download(img.data(), n, stream_);
-  if (o.tags) tag_.download(o.tags, n, stream_);
-  if (o.molecule_ids) molid_.download(o.molecule_ids, n, stream_);
-  synchronize();
-  for (size_t i = 0; i < n; ++i) {
-    if (o.positions) {
-      o.positions[3 * i] = pos[i].x;
-      o.positions[3 * i + 1] = pos[i].y;
-      o.positions[3 * i + 2] = pos[i].z;
-    }
-    if (o.types) o.types[i] = static_cast<int32_t>(id_of(pos[i].w)) + 1;
-    if (o.velocities) {
-      o.velocities[3 * i] = vel[i].x;
-      o.velocities[3 * i + 1] = vel[i].y;
-      o.velocities[3 * i + 2] = vel[i].z;
-    }
-    if (o.masses) o.masses[i] = vel[i].w;
-    if (o.forces) {
-      o.forces[3 * i] = force[i].x;
-      o.forces[3 * i + 1] = force[i].y;
-      o.forces[3 * i + 2] = force[i].z;
-    }
-    if (o.images) {
-      o.images[3 * i] = img[i].x;
-      o.images[3 * i + 1] = img[i].y;
-      o.images[3 * i + 2] = img[i].z;
-    }
-  }
+  StateSource src;
+  src.n = n_;
+  src.pos = pos_.data();
+  src.vel = vel_.data();
+  src.force = force_.data();
+  src.image = image_.data();
+  src.tag = tag_.data();
+  src.molid = molid_.data();
+  state_reader_.read(src, o, stream_);
+  if (frame_mode_) check_overflow(fetch_ctrl());
 }
 
 void Engine::read_neighbors(uint32_t* counts, uint32_t* list, uint64_t capacity) {

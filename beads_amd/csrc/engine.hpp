@@ -15,6 +15,7 @@
 #include "kernels.hpp"
 #include "models.hpp"
 #include "output.hpp"
+#include "state_reader.hpp"
 
 namespace beads_amd {
 
@@ -202,6 +203,7 @@ class Engine {
   DeviceBuffer<double> partials_;
   DeviceBuffer<double> pair_acc_;  // half list: partner-side LJ sums [3 N]
 
+  StateReader state_reader_;
   DeviceBuffer<Ctrl> ctrl_;
   DeviceBuffer<unsigned long long> neighbor_parts_;
   DeviceBuffer<uint64_t> sync_lines_;  // rebuild_kernel's meeting points

@@ -457,6 +457,46 @@ __global__ __launch_bounds__(kBlock) void pack_records_kernel(PackParams p) {
   }
 }
 
+// The wanted fields of every atom, each an array of its own (a host copy of
+// whole records would leave the taking apart, and a quarter more bytes, to one
+// host thread).
+__global__ __launch_bounds__(kBlock) void pack_state_kernel(PackStateParams p) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= p.n) {
+    return;
+  }
+  auto put3 = [&](uint64_t field, auto x, auto y, auto z) {
+    auto* o = reinterpret_cast<decltype(x)*>(p.out + field) + 3 * static_cast<size_t>(i);
+    o[0] = x;
+    o[1] = y;
+    o[2] = z;
+  };
+  if (p.positions != kNoField || p.types != kNoField) {
+    const real4 x = p.pos[i];
+    if (p.positions != kNoField) put3(p.positions, x.x, x.y, x.z);
+    if (p.types != kNoField) {
+      reinterpret_cast<int32_t*>(p.out + p.types)[i] = static_cast<int32_t>(id_of(x.w)) + 1;
+    }
+  }
+  if (p.velocities != kNoField || p.masses != kNoField) {
+    const real4 v = p.vel[i];
+    if (p.velocities != kNoField) put3(p.velocities, v.x, v.y, v.z);
+    if (p.masses != kNoField) reinterpret_cast<real_t*>(p.out + p.masses)[i] = v.w;
+  }
+  if (p.forces != kNoField) {
+    const real4 f = p.force[i];
+    put3(p.forces, f.x, f.y, f.z);
+  }
+  if (p.images != kNoField) {
+    const int4 m = p.image[i];
+    put3(p.images, m.x, m.y, m.z);
+  }
+  if (p.tags != kNoField) reinterpret_cast<uint32_t*>(p.out + p.tags)[i] = p.tag[i];
+  if (p.molecule_ids != kNoField) {
+    reinterpret_cast<uint32_t*>(p.out + p.molecule_ids)[i] = p.molid[i];
+  }
+}
+
 // cell_list_build.cu:183-219: gather every per-atom array into cell order
 // (new slot s takes old slot cell_atoms[s]) and record the inverse map.
 __device__ __forceinline__ void gather_atom(const ReorderParams& p, uint32_t s) {
@@ -1473,6 +1513,10 @@ void launch_pack_records(const PackParams& p, hipStream_t stream) {
 // of 32,000 64 / 38, of 108,000 97 / 83, of 256,000 157 / 171; four-type
 // mixture of 64,000 62 / 56, of 100,000 75 / 76, of 216,000 119 / 139.
 constexpr uint32_t kWideBuildMax = 100000;
+
+void launch_pack_state(const PackStateParams& p, hipStream_t stream) {
+  pack_state_kernel<<<grid_for(p.n), kBlock, 0, stream>>>(p);
+}
 
 void launch_build(const BuildParams& params, hipStream_t stream) {
   const unsigned g = grid_for(params.n, kBuildAtoms);

@@ -88,6 +88,22 @@ struct PackParams {
 };
 void launch_pack_records(const PackParams& p, hipStream_t stream);
 
+// The state as arrays of one field each: byte offsets into out (kNoField: not
+// wanted).
+constexpr uint64_t kNoField = ~uint64_t{0};
+struct PackStateParams {
+  uint32_t n;
+  const real4* pos;
+  const real4* vel;
+  const real4* force;
+  const int4* image;
+  const uint32_t* tag;
+  const uint32_t* molid;
+  unsigned char* out;
+  uint64_t positions, velocities, forces, masses, images, types, tags, molecule_ids;
+};
+void launch_pack_state(const PackStateParams& p, hipStream_t stream);
+
 // One step's work.
 void launch_force(const ForceParams& p, bool kick, bool observables, hipStream_t stream);
 void launch_integrate(const IntegrateParams& p, bool thermostat, bool check,
