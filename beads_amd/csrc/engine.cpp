@@ -602,7 +602,7 @@ void Engine::upload_state() {
   upload_parameters();
 
   // Per-workgroup partial sums of the force pass (the widest grid) and of scale.
-  partials_.resize(9 * static_cast<size_t>(std::max(force_grid(n_), grid_for(n_))));
+  partials_.resize(9 * static_cast<size_t>(grid_for(n_, kBlock / kForceTeamMax)));
   if (half_list_) {
     pair_acc_.resize(3 * n);
     pair_acc_.zero(stream_);

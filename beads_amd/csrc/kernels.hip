@@ -1,7 +1,7 @@
 // gfx950 kernels of the per-step MD path.
 //
 // Design (CDNA4): 256-wide workgroups (4 wave64s), one work-item per atom
-// except in the force pass (a team of kTeam lanes per atom), real4 SoA
+// except in the force pass and the build (a team of lanes per atom), real4 SoA
 // streams (float4, or double4 in the BEADS_REAL64 build), FP64 for LJ pair
 // values and global reductions. Kernels that gather
 // neighbour positions map workgroups onto atoms XCD by XCD so each XCD's L2
@@ -1110,17 +1110,17 @@ __device__ __forceinline__ void lj_list(const ForceParams& p, uint32_t i, real4 
   }
 }
 
-// LJ over atom i's stored list, shared by the kTeam lanes of its team: lane t
-// takes slots base + u*kTeam + t, u < kTeamSlots, and keeps FP64 partial sums
+// LJ over atom i's stored list, shared by the TEAM lanes of its team: lane t
+// takes slots base + u*TEAM + t, u < SLOTS, and keeps FP64 partial sums
 // (pair_lj.cu:21-167; same decision and pair value as lj_list). Slots at or
 // past cnt neither load an index nor count; they gather atom i itself.
-template <bool OBS, int TYPES>
+template <bool OBS, int TYPES, int TEAM, int SLOTS>
 __device__ __forceinline__ void lj_team(const ForceParams& p, uint32_t i, uint32_t t, real4 xi4,
                                         const LjCoeff* lj_lds, const LjCoeff& c0, double& fxd,
                                         double& fyd, double& fzd, double& e_pair,
                                         double& w_pair) {
-  static_assert(kNbrChunk % kTeam == 0, "a team's slots of one round share a chunk");
-  static_assert(kTeam * kTeamSlots == kNbrRound, "a round covers the padded capacity's unit");
+  static_assert(kNbrChunk % TEAM == 0, "a team's slots of one load share a chunk");
+  static_assert(kNbrRound % (TEAM * SLOTS) == 0, "a round stays inside the padded capacity");
   const int T = p.n_types;
   const int ti = static_cast<int>(id_of(xi4.w));
   const uint32_t n = p.n;
@@ -1128,32 +1128,32 @@ __device__ __forceinline__ void lj_team(const ForceParams& p, uint32_t i, uint32
   const real_t h0 = p.box.hL[0], h1 = p.box.hL[1], h2 = p.box.hL[2];
   const real_t xm0 = xi4.x - L0, xm1 = xi4.y - L1, xm2 = xi4.z - L2;
   const uint32_t cnt = p.nbr_count[i];
-  for (uint32_t base = 0; base < cnt; base += kTeam * kTeamSlots) {
+  for (uint32_t base = 0; base < cnt; base += TEAM * SLOTS) {
     // Every slot of the round lies inside the atom's padded capacity; slots
     // at or past the count read whatever the chunk holds and become i.
-    uint32_t jj[kTeamSlots];
+    uint32_t jj[SLOTS];
 #pragma unroll
-    for (int u = 0; u < kTeamSlots; ++u) {
-      const uint32_t s = base + u * kTeam + t;
+    for (int u = 0; u < SLOTS; ++u) {
+      const uint32_t s = base + u * TEAM + t;
       jj[u] = p.nbr[nbr_chunk_base(s / kNbrChunk, i, n) + (s & (kNbrChunk - 1))];
     }
-    // slot base + u * kTeam + t holds a neighbour iff u * kTeam < rem
+    // slot base + u * TEAM + t holds a neighbour iff u * TEAM < rem
     const int rem = static_cast<int>(cnt) - static_cast<int>(base + t);
 #pragma unroll
-    for (int u = 0; u < kTeamSlots; ++u) {
-      jj[u] = u * kTeam < rem ? jj[u] : i;
+    for (int u = 0; u < SLOTS; ++u) {
+      jj[u] = u * TEAM < rem ? jj[u] : i;
     }
     // Gathers as a 32-bit byte offset from the array base (n * sizeof(real4)
     // < 2^32, checked at set-up).
     const char* pos_bytes = reinterpret_cast<const char*>(p.pos);
-    real4 xj[kTeamSlots];
+    real4 xj[SLOTS];
 #pragma unroll
-    for (int u = 0; u < kTeamSlots; ++u) {
+    for (int u = 0; u < SLOTS; ++u) {
       xj[u] = *reinterpret_cast<const real4*>(
           pos_bytes + jj[u] * static_cast<uint32_t>(sizeof(real4)));
     }
 #pragma unroll
-    for (int u = 0; u < kTeamSlots; ++u) {
+    for (int u = 0; u < SLOTS; ++u) {
       // mic_diff_sel returns the raw difference unless it exceeds half the
       // box; the folded forms are formed only when some lane of the wave
       // needs them (pairs across a periodic boundary), the same values.
@@ -1167,7 +1167,7 @@ __device__ __forceinline__ void lj_team(const ForceParams& p, uint32_t i, uint32
         dz = mic_diff_sel(xi4.z, xm2, xj[u].z, L2, h2);
       }
       const real_t r2 = r2_strict(dx, dy, dz);
-      if (u * kTeam < rem && r2 < p.rc2) {
+      if (u * TEAM < rem && r2 < p.rc2) {
         LjCoeff c;
         if (TYPES == 0) {
           c = c0;
@@ -1342,20 +1342,20 @@ __global__ __launch_bounds__(kReduceBlock) void step_reduce_kernel(ForceParams p
 // reduction for the Berendsen factor (berendsen_thermostat.cu:109-163) as
 // per-workgroup partials, which step_reduce_kernel totals in FP64.
 //
-// Each atom has a team of kTeam adjacent lanes. Lane t reads list slots
-// base + u*kTeam + t (u < kTeamSlots), so one gather instruction fetches
-// kTeam consecutive entries of each of the wave's 64/kTeam lists: mostly
+// Each atom has a team of TEAM adjacent lanes. Lane t reads list slots
+// base + u*TEAM + t (u < SLOTS), so one gather instruction fetches
+// TEAM consecutive entries of each of the wave's 64/TEAM lists: mostly
 // consecutive slots of one cell, a few cache lines per atom instead of one
 // line per lane. The team's FP64 partial sums meet in a shuffle butterfly and
 // the atom's total is rounded to binary32 once.
-template <bool KICK, bool OBS, int TYPES, bool HALF, bool SPILL>
+template <bool KICK, bool OBS, int TYPES, bool HALF, bool SPILL, int TEAM, int SLOTS>
 __global__ __launch_bounds__(kBlock) void force_kernel(ForceParams p) {
   __shared__ LjCoeff lj_lds[TYPES == 1 && !HALF ? kMaxLdsTypes * kMaxLdsTypes : 1];
   __shared__ double red_lds[4];
   if (!HALF) load_lj_table<TYPES>(p, lj_lds);
   const LjCoeff c0 = TYPES == 0 && !HALF ? p.lj[0] : LjCoeff{0.0, 0.0, 0.0, 0.0};
-  const uint32_t t = threadIdx.x & (kTeam - 1);
-  const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * kForceAtoms + threadIdx.x / kTeam;
+  const uint32_t t = threadIdx.x & (TEAM - 1);
+  const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * (kBlock / TEAM) + threadIdx.x / TEAM;
   StepSums sums;
   if (i < p.n) {  // uniform over a team
     const real4 xi4 = p.pos[i];
@@ -1371,14 +1371,14 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceParams p) {
         acc[2] = 0.0;
       }
     } else {
-      lj_team<OBS, TYPES>(p, i, t, xi4, lj_lds, c0, fxd, fyd, fzd, sums.e_pair, sums.w_pair);
+      lj_team<OBS, TYPES, TEAM, SLOTS>(p, i, t, xi4, lj_lds, c0, fxd, fyd, fzd, sums.e_pair, sums.w_pair);
     }
     if (p.topo.has_listed) {
-      listed_team<OBS, SPILL, kTeam>(p.pos, p.topo, p.box, p.n, i, t, xi4, fxd, fyd, fzd, sums);
+      listed_team<OBS, SPILL, TEAM>(p.pos, p.topo, p.box, p.n, i, t, xi4, fxd, fyd, fzd, sums);
     }
-    fxd = team_sum<kTeam>(fxd);
-    fyd = team_sum<kTeam>(fyd);
-    fzd = team_sum<kTeam>(fzd);
+    fxd = team_sum<TEAM>(fxd);
+    fyd = team_sum<TEAM>(fyd);
+    fzd = team_sum<TEAM>(fzd);
     if (t == 0) {
       finish_atom<KICK>(p, i, fxd, fyd, fzd, sums);
     }
@@ -1556,6 +1556,25 @@ void launch_build(const BuildParams& params, hipStream_t stream) {
 #undef BEADS_BUILD_CASE
 }
 
+// Lanes per atom and slots per lane of the force pass. Four lanes an atom cost
+// least per slot and per listed term; below some tens of thousands of atoms
+// they leave the GPU too few waves, and the pass lasts as long as one atom's
+// chain of rounds and terms, which more lanes shorten. Measured 4x8 / 8x4 /
+// 16x2, us per pass: LJ fluid of 500 beads 8.7 / 6.7 / 5.4, of 4,000
+// 8.6 / 6.3 / 5.4, of 32,000 10.1 / 9.0 / 10.2; bead-spring melt of 8,000
+// 14.2 / 10.7 / 10.7, of 18,000 16.8 / 14.6 / 14.8, of 48,000
+// 22.5 / 23.1 / 29.1; mixture of 8,000 8.9 / 7.7 / 5.9, of 64,000
+// 13.9 / 14.3 / 16.7. More slots in flight (8x8, 16x4, 16x8) gain at most 0.5
+// us and would widen the lists' padding.
+constexpr uint32_t kForceTeam16Max = 12000;
+constexpr uint32_t kForceTeam8Max = 40000;
+
+static ForceShape force_shape(uint32_t n) {
+  if (n <= kForceTeam16Max) return {16, 2};
+  if (n <= kForceTeam8Max) return {8, 4};
+  return {4, 8};
+}
+
 void launch_force(const ForceParams& p, bool kick, bool obs, hipStream_t stream) {
   const unsigned g = grid_for(p.n);
   const int types = p.n_types == 1 ? 0 : (p.n_types <= kMaxLdsTypes ? 1 : 2);
@@ -1571,22 +1590,30 @@ void launch_force(const ForceParams& p, bool kick, bool obs, hipStream_t stream)
     BEADS_HALF_CASE(true, 2)
 #undef BEADS_HALF_CASE
   }
-  const unsigned gf = force_grid(p.n);
   const bool spill = p.topo.spill_index != nullptr;
+  // The half list's and the spill's variants exist in the widest-work shape only.
+  const ForceShape shape = half || spill ? ForceShape{4, 8} : force_shape(p.n);
+  const unsigned gf = grid_for(p.n, kBlock / shape.team);
+#define BEADS_FORCE_SHAPE(K, O, T, N, S)                                               \
+  if (shape.team == N && shape.slots == S) {                                           \
+    force_kernel<K, O, T, false, false, N, S><<<gf, kBlock, 0, stream>>>(p);           \
+  }
 #define BEADS_FORCE_CASE(K, O, T)                                                      \
   if (kick == K && obs == O && (half || types == T)) {                                 \
     if (half) {                                                                        \
       if (spill) {                                                                     \
-        force_kernel<K, O, 0, true, true><<<gf, kBlock, 0, stream>>>(p);               \
+        force_kernel<K, O, 0, true, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);         \
       } else {                                                                         \
-        force_kernel<K, O, 0, true, false><<<gf, kBlock, 0, stream>>>(p);              \
+        force_kernel<K, O, 0, true, false, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
       }                                                                                \
       step_reduce_kernel<K, O, true><<<1, kReduceBlock, 0, stream>>>(p, gf);           \
     } else {                                                                           \
       if (spill) {                                                                     \
-        force_kernel<K, O, T, false, true><<<gf, kBlock, 0, stream>>>(p);              \
+        force_kernel<K, O, T, false, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
       } else {                                                                         \
-        force_kernel<K, O, T, false, false><<<gf, kBlock, 0, stream>>>(p);             \
+        BEADS_FORCE_SHAPE(K, O, T, 4, 8)                                               \
+        BEADS_FORCE_SHAPE(K, O, T, 8, 4)                                               \
+        BEADS_FORCE_SHAPE(K, O, T, 16, 2)                                              \
       }                                                                                \
       step_reduce_kernel<K, O, false><<<1, kReduceBlock, 0, stream>>>(p, gf);          \
     }                                                                                  \
@@ -1605,6 +1632,7 @@ void launch_force(const ForceParams& p, bool kick, bool obs, hipStream_t stream)
   BEADS_FORCE_CASE(false, true, 1)
   BEADS_FORCE_CASE(false, true, 2)
 #undef BEADS_FORCE_CASE
+#undef BEADS_FORCE_SHAPE
 }
 
 void launch_integrate(const IntegrateParams& p, bool thermostat, bool check,

@@ -48,14 +48,12 @@ inline unsigned grid_for(uint32_t n, int block = kBlock) {
   return static_cast<unsigned>((static_cast<uint64_t>(n) + block - 1) / block);
 }
 
-// The force pass gives every atom a team of kTeam adjacent lanes; each lane
-// takes kTeamSlots neighbour slots per round. A workgroup covers kForceAtoms
-// atoms.
-constexpr int kTeam = 4;
-constexpr int kTeamSlots = 8;
-constexpr int kForceAtoms = kBlock / kTeam;
-
-inline unsigned force_grid(uint32_t n) { return grid_for(n, kForceAtoms); }
+// The force pass gives every atom a team of adjacent lanes; each lane takes
+// `slots` neighbour slots per round.
+struct ForceShape {
+  int team, slots;
+};
+constexpr int kForceTeamMax = 16;
 
 // Entries allocated past the last atom in the build's candidate streams (the
 // position array and its cell-ordered copy): a build round loads 16
