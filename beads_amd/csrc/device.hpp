@@ -155,6 +155,7 @@ struct ForceParams {
   double dt_over_tau;
   double dof;
   double* partials;       // per block: ke, pe[4], vir[4]
+  int32_t sums;           // form them (set by launch_force)
   Ctrl* ctrl;
   uint32_t* cell_count;   // zeroed after a rebuild consumed it
   uint32_t n_cells;

@@ -800,8 +800,8 @@ void Engine::rebuild_sequence(bool forced, uint64_t steps) {
   launch_build(build_params_, stream_);
 }
 
-void Engine::force_pass(bool kick, bool observables) {
-  launch_force(force_params_, kick, observables, stream_);
+void Engine::force_pass(bool kick, bool observables, bool sums) {
+  launch_force(force_params_, kick, observables, sums, stream_);
 }
 
 void Engine::initialize(bool observables) {
@@ -816,7 +816,7 @@ void Engine::initialize(bool observables) {
 // SimulationRun::advance_dynamics_step (simulation_run.cpp:212-235): pending
 // thermostat factor + pre-force, neighbour update, forces + post-force +
 // Berendsen factor.
-void Engine::step_once(bool observables) {
+void Engine::step_once(bool observables, bool more) {
   const uint64_t physical = step_ + 1;
   const bool every = plan_.cutoff_buffer == 0.f;
   const bool check = !every && physical % plan_.check_every == 0;
@@ -824,7 +824,11 @@ void Engine::step_once(bool observables) {
   if (every || check) {
     rebuild_sequence(every, every ? uint64_t{1} : plan_.check_every);
   }
-  force_pass(true, observables);
+  // Without a thermostat the kinetic energy of a step is read only by the host,
+  // after the call's last step: the reduction, a quarter of a 4,000-bead
+  // fluid's launches, is left to that one. (The half list's pair sums are
+  // cleared by it.)
+  force_pass(true, observables, observables || thermostat_ || half_list_ || !more);
   ke_from_scale_ = false;
   step_ = physical;
 }
@@ -844,7 +848,7 @@ void Engine::replay_step_graph() {
   if (step_graph_exec_ == nullptr) {
     const uint64_t saved = step_;
     BEADS_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-    for (uint64_t k = 0; k < g; ++k) step_once(false);
+    for (uint64_t k = 0; k < g; ++k) step_once(false, k + 1 < g);
     hipGraph_t graph = nullptr;
     BEADS_HIP(hipStreamEndCapture(stream_, &graph));
     BEADS_HIP(hipGraphInstantiate(&step_graph_exec_, graph, nullptr, nullptr, 0));
@@ -868,7 +872,7 @@ void Engine::advance(uint64_t n_steps, bool observables_on_last) {
       left -= g;
       continue;
     }
-    step_once(observables_on_last && left == 1);
+    step_once(observables_on_last && left == 1, left > 1);
     --left;
   }
   BEADS_HIP(hipGetLastError());

@@ -140,8 +140,9 @@ class Engine {
   void set_up_params();
   // steps: steps advanced since the previous rebuild sequence (0 at set-up).
   void rebuild_sequence(bool forced, uint64_t steps);
-  void force_pass(bool kick, bool observables);
-  void step_once(bool observables);
+  void force_pass(bool kick, bool observables, bool sums = true);
+  // more: another step of the same call follows, whatever the host does.
+  void step_once(bool observables, bool more = false);
   uint64_t graph_steps() const;
   void replay_step_graph();
   void materialize_velocities();

@@ -1275,8 +1275,8 @@ __device__ __forceinline__ void store_step_partials(const ForceParams& p, const 
 }
 
 // One workgroup after the force pass: FP64 totals of the nbk workgroups'
-// partials, the Berendsen factor (berendsen_thermostat.cu:109-163), and the
-// per-step flags cleared. A kernel of its own, so the force pass publishes
+// partials and the Berendsen factor (berendsen_thermostat.cu:109-163). Steps
+// whose sums nobody reads (ForceParams::sums) do without it. A kernel of its own, so the force pass publishes
 // its partials at the kernel boundary instead of with a device-scope fence
 // (an L2 write-back and invalidate on gfx950) in every workgroup.
 constexpr int kReduceBlock = 1024;
@@ -1341,12 +1341,9 @@ __global__ __launch_bounds__(kReduceBlock) void step_reduce_kernel(ForceParams p
       ctrl->virial[q - 5] = (HALF && q == 5) ? ctrl->half_pair[1] : acc;
     }
   }
-  if (HALF) __syncthreads();  // half_pair is read before it is cleared
-  if (threadIdx.x == 0) {
-    p.ctrl->rebuild = 0;
-    p.ctrl->reorder = 0;
-    p.ctrl->joined = 0;
-    if (HALF) {
+  if (HALF) {
+    __syncthreads();  // half_pair is read before it is cleared
+    if (threadIdx.x == 0) {
       p.ctrl->half_pair[0] = 0.0;
       p.ctrl->half_pair[1] = 0.0;
     }
@@ -1370,6 +1367,11 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceParams p) {
   __shared__ LjCoeff lj_lds[TYPES == 1 && !HALF ? kMaxLdsTypes * kMaxLdsTypes : 1];
   __shared__ double red_lds[4];
   if (!HALF) load_lj_table<TYPES>(p, lj_lds);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // the step's rebuild is done
+    p.ctrl->rebuild = 0;
+    p.ctrl->reorder = 0;
+    p.ctrl->joined = 0;
+  }
   const LjCoeff c0 = TYPES == 0 && !HALF ? p.lj[0] : LjCoeff{0.0, 0.0, 0.0, 0.0};
   const uint32_t t = threadIdx.x & (TEAM - 1);
   const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * (kBlock / TEAM) + threadIdx.x / TEAM;
@@ -1400,7 +1402,7 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceParams p) {
       finish_atom<KICK>(p, i, fxd, fyd, fzd, sums);
     }
   }
-  store_step_partials<OBS>(p, sums, red_lds);
+  if (p.sums) store_step_partials<OBS>(p, sums, red_lds);
 }
 
 // Apply the pending Berendsen factor and reduce the kinetic energy of the
@@ -1594,7 +1596,9 @@ static ForceShape force_shape(uint32_t n) {
   return {4, 8};
 }
 
-void launch_force(const ForceParams& p, bool kick, bool obs, hipStream_t stream) {
+void launch_force(const ForceParams& params, bool kick, bool obs, bool sums, hipStream_t stream) {
+  ForceParams p = params;
+  p.sums = sums ? 1 : 0;
   const unsigned g = grid_for(p.n);
   const int types = p.n_types == 1 ? 0 : (p.n_types <= kMaxLdsTypes ? 1 : 2);
   const bool half = p.half != 0;
@@ -1625,7 +1629,7 @@ void launch_force(const ForceParams& p, bool kick, bool obs, hipStream_t stream)
       } else {                                                                         \
         force_kernel<K, O, 0, true, false, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
       }                                                                                \
-      step_reduce_kernel<K, O, true><<<1, kReduceBlock, 0, stream>>>(p, gf);           \
+      if (sums) step_reduce_kernel<K, O, true><<<1, kReduceBlock, 0, stream>>>(p, gf); \
     } else {                                                                           \
       if (spill) {                                                                     \
         force_kernel<K, O, T, false, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
@@ -1634,7 +1638,7 @@ void launch_force(const ForceParams& p, bool kick, bool obs, hipStream_t stream)
         BEADS_FORCE_SHAPE(K, O, T, 8, 4)                                               \
         BEADS_FORCE_SHAPE(K, O, T, 16, 2)                                              \
       }                                                                                \
-      step_reduce_kernel<K, O, false><<<1, kReduceBlock, 0, stream>>>(p, gf);          \
+      if (sums) step_reduce_kernel<K, O, false><<<1, kReduceBlock, 0, stream>>>(p, gf); \
     }                                                                                  \
     return;                                                                            \
   }

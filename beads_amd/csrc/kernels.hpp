@@ -103,7 +103,10 @@ struct PackStateParams {
 void launch_pack_state(const PackStateParams& p, hipStream_t stream);
 
 // One step's work.
-void launch_force(const ForceParams& p, bool kick, bool observables, hipStream_t stream);
+// sums: total the kinetic energy (with observables also energies and virials)
+// and form the Berendsen factor.
+void launch_force(const ForceParams& p, bool kick, bool observables, bool sums,
+                  hipStream_t stream);
 void launch_integrate(const IntegrateParams& p, bool thermostat, bool check,
                       bool force_rebuild, hipStream_t stream);
 void launch_scale(const ScaleParams& p, bool thermostat, hipStream_t stream);
