@@ -275,8 +275,8 @@ constexpr int kRunCodeShift = 28;
 constexpr uint32_t kRunIndexMask = (1u << kRunCodeShift) - 1u;
 
 // The runs of row r (z neighbour r / 3, y neighbour r % 3) of an atom at xi in
-// cell (cx, cy, cz); empty runs are {0, 0}. With 5 or more cells per axis a
-// row whose cells lie at least gy along y and gz along z from the atom holds
+// cell (cx, cy, cz); empty runs are {0, 0}. PRUNE, with 5 or more cells per
+// axis: a row whose cells lie at least gy along y and gz along z from the atom holds
 // neighbours only within ext = sqrt(r_s^2 - gy^2 - gz^2) along x, and none when
 // gy^2 + gz^2 > r_s^2: such rows are dropped, and with x-bin tables (xbins,
 // members of a cell ascending in x) the row starts and ends at the bins within
@@ -284,10 +284,12 @@ constexpr uint32_t kRunIndexMask = (1u << kRunCodeShift) - 1u;
 // cell). The gaps are taken kGapSlack of a cell short, far above the rounding
 // of the cell coordinates, so a skipped member is farther than ext along x, or
 // than the gaps along y and z, by a margin that no rounding of r^2 closes: the
-// accepted candidates and their order are those of the full scan.
+// accepted candidates and their order are those of the full scan (of atoms
+// inside the box, as the wrap leaves them; without PRUNE of any).
 struct RunPair {
   uint2 a, b;
 };
+template <bool PRUNE>
 __device__ inline RunPair row_run_pair(const CellGridView& g, const BoxView& box, real_t rs2,
                                        const uint32_t* cell_start, const uint4* xbins, real4 xi,
                                        uint32_t cx, uint32_t cy, uint32_t cz, uint32_t r) {
@@ -325,7 +327,7 @@ __device__ inline RunPair row_run_pair(const CellGridView& g, const BoxView& box
   uint32_t skip = 0, keep = 0xffffffffu;  // members dropped at the row's start, kept of its last cell
   uint32_t n_last = 0;
   const uint32_t last = rowc + (m1 >= m0 ? m1 : l1);
-  if (g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
+  if (PRUNE && g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
     constexpr real_t kGapSlack = static_cast<real_t>(1.0 / 64.0);
     const real_t fy = (xi.y - box.lo[1]) * g.inv_cell[1] - static_cast<real_t>(cy);
     const real_t fz = (xi.z - box.lo[2]) * g.inv_cell[2] - static_cast<real_t>(cz);
@@ -372,7 +374,7 @@ __device__ inline RunPair row_run_pair(const CellGridView& g, const BoxView& box
 // A team's runs in visiting order, empty ones left out, into its LDS entry
 // list (kMaxRuns entries); returns how many, the same in every lane. Lane t of
 // TEAM evaluates rows t, t + TEAM, ... Every lane of the team calls it.
-template <int TEAM>
+template <int TEAM, bool PRUNE>
 __device__ inline uint32_t team_runs(const CellGridView& g, const BoxView& box, real_t rs2,
                                      const uint32_t* cell_start, const uint4* xbins, real4 xi,
                                      uint32_t c, uint32_t t, uint32_t team_lane0, uint2* runs) {
@@ -384,7 +386,7 @@ __device__ inline uint32_t team_runs(const CellGridView& g, const BoxView& box, 
     RunPair p;
     p.a = p.b = make_uint2(0u, 0u);
     if (r0 + t < static_cast<uint32_t>(kRows)) {
-      p = row_run_pair(g, box, rs2, cell_start, xbins, xi, cx, cy, cz, r0 + t);
+      p = row_run_pair<PRUNE>(g, box, rs2, cell_start, xbins, xi, cx, cy, cz, r0 + t);
     }
     const bool has_a = p.a.y != 0, has_b = p.b.y != 0;  // a nonempty run ends past 0
     const uint64_t ma = (__ballot(has_a) >> team_lane0) & kTeamMask;
@@ -415,9 +417,10 @@ template <int TEAM, int SLOTS, typename Entry, typename Accept, typename Put, ty
 __device__ __forceinline__ uint32_t scan_runs(const uint2* runs, uint32_t n_runs, uint32_t t,
                                               uint32_t team_lane0, const BoxView& box, Entry entry,
                                               Accept accept, Put put, Mode mode) {
+  static_assert(TEAM <= 32, "a team's lane mask is one word");
   constexpr uint32_t kRound = TEAM * SLOTS;
-  constexpr uint64_t kTeamMask = TEAM >= 64 ? ~0ull : (1ull << TEAM) - 1ull;
-  const uint64_t below = (1ull << t) - 1ull;
+  constexpr uint32_t kTeamMask = static_cast<uint32_t>((1ull << TEAM) - 1ull);
+  const uint32_t below = (1u << t) - 1u;
   uint32_t count = 0;
   if (n_runs == 0) return count;
   uint32_t r = 0, k, e;
@@ -458,11 +461,11 @@ __device__ __forceinline__ uint32_t scan_runs(const uint2* runs, uint32_t n_runs
     for (int u = 0; u < SLOTS; ++u) {
       const uint32_t j = id_of(x[u].w);
       const uint64_t m = __builtin_amdgcn_ballot_w64(u * TEAM < left) & accept(j, x[u], mode, shift);
-      const uint64_t bits = (m >> team_lane0) & kTeamMask;
+      const uint32_t bits = static_cast<uint32_t>(m >> team_lane0) & kTeamMask;
       if (__builtin_amdgcn_inverse_ballot_w64(m)) {
-        put(count + static_cast<uint32_t>(__builtin_popcountll(bits & below)), j);
+        put(count + static_cast<uint32_t>(__builtin_popcount(bits & below)), j);
       }
-      count += static_cast<uint32_t>(__builtin_popcountll(bits));
+      count += static_cast<uint32_t>(__builtin_popcount(bits));
     }
     if (!more) break;
   }

@@ -648,7 +648,7 @@ __device__ inline bool row_runs(const BuildParams& p, uint32_t i, uint32_t t, ui
 #pragma unroll 1
   for (uint32_t r = t; r < static_cast<uint32_t>(kRows); r += kBuildTeam) {
     const uint2 d =
-        row_run_pair(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r).a;
+        row_run_pair<true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r).a;
     rows[r] = d;
     const uint32_t b = d.x, e = d.y & kRunIndexMask;
     if (b < e) {
@@ -928,7 +928,7 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
 #pragma unroll 1
         for (uint32_t r = 0; r < static_cast<uint32_t>(kRows); ++r) {
           const RunPair q =
-              row_run_pair(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r);
+              row_run_pair<true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r);
 #pragma unroll 1
           for (int part = 0; part < 2; ++part) {
             const uint2 d = part == 0 ? q.a : q.b;
@@ -992,7 +992,7 @@ __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
     } else {
       xi = p.cell_pos[q];  // the atom's position, .w its slot
       i = id_of(xi.w);
-      n_runs = team_runs<kWideTeam>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi,
+      n_runs = team_runs<kWideTeam, true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi,
                                     cell_of_position(xi, p.box, g), t, team_lane0, runs);
     }
   }

@@ -800,17 +800,18 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_reorder_commit_kernel(Rep
 // a team of kPhasedBuildTeam adjacent lanes per atom. The candidates are
 // build_atom's in its order (neighbour cells in neighbourhood order, a cell's
 // members in slot order, read from the cell-ordered positions; every atom on
-// the direct path), as runs of the cell-ordered stream (team_runs), less the
-// rows of cells that lie beyond r_s, whose members build_atom rejects; the team
+// the direct path), as runs of the cell-ordered stream (team_runs); the team
 // appends the accepted ones in candidate order through a ballot (scan_runs), so
-// the lists are build_atom's. A replica's overflow is the OR over its chunks.
+// the lists are build_atom's, also of a replica whose atoms have left the box
+// (no row is dropped by its distance, and every candidate takes the minimum
+// image). A replica's overflow is the OR over its chunks.
 // Bound by one atom's chain of runs: a step rebuilds a few replicas, too few
-// atoms to fill the GPU, so an atom takes a quarter wave, whose round covers a
-// row of cells. With four lanes per atom and one run per cell, 27 bounds and
-// twice as many rounds one after another, builds took 99 us per step of 64
-// LJ replicas (about 300,000 beads) and now take 70 (24 melts: 82 and 31).
+// atoms to fill the GPU, so an atom takes a quarter wave. With four lanes per
+// atom and one run per cell, 27 bounds and twice as many rounds one after
+// another, builds took 99 us per step of 64 LJ replicas (about 400,000 beads)
+// and now take 66 (24 melts: 82 and 32).
 constexpr int kPhasedBuildTeam = 16;
-constexpr int kPhasedBuildSlots = 4;
+constexpr int kPhasedBuildSlots = 2;
 constexpr uint32_t kPhasedBuildAtoms = kPhasedBlock / kPhasedBuildTeam;
 constexpr uint32_t kBuildParts = kReplicaChunk / kPhasedBuildAtoms;  // workgroups per chunk
 
@@ -841,7 +842,7 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_build_kernel(ReplicaParam
         if (t == 0) runs[0] = make_uint2(0u, n);
         n_runs = 1;
       } else {
-        n_runs = team_runs<kPhasedBuildTeam>(g, d.box, d.rs2, A.cell_start + d.cell0, nullptr, xi,
+        n_runs = team_runs<kPhasedBuildTeam, false>(g, d.box, d.rs2, A.cell_start + d.cell0, nullptr, xi,
                                              A.cell_of[d.atom0 + i], t, team_lane0, runs);
       }
     }
@@ -861,17 +862,10 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_build_kernel(ReplicaParam
                     ? excl[static_cast<size_t>(k) * n + i]
                     : 0xffffffffu;
       }
-      const auto accept = [&](uint32_t j, real4 xj, auto mode, real3 sh) -> uint64_t {
-        real_t dx, dy, dz;
-        if (decltype(mode)::value == kGeneric) {
-          dx = mic(xi.x - xj.x, L0, h0);
-          dy = mic(xi.y - xj.y, L1, h1);
-          dz = mic(xi.z - xj.z, L2, h2);
-        } else {
-          dx = (xi.x - xj.x) + sh.x;
-          dy = (xi.y - xj.y) + sh.y;
-          dz = (xi.z - xj.z) + sh.z;
-        }
+      const auto accept = [&](uint32_t j, real4 xj, auto, real3) -> uint64_t {
+        const real_t dx = mic(xi.x - xj.x, L0, h0);
+        const real_t dy = mic(xi.y - xj.y, L1, h1);
+        const real_t dz = mic(xi.z - xj.z, L2, h2);
         uint64_t m = __builtin_amdgcn_ballot_w64(!(r2_strict(dx, dy, dz) > rs2)) &
                      __builtin_amdgcn_ballot_w64(j != i);
         if (EXCL > 0) {
@@ -897,13 +891,8 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_build_kernel(ReplicaParam
       } else {
         const real4* cpos = A.cell_pos + d.atom0;
         const auto entry = [cpos](uint32_t k) { return cpos[k]; };
-        if (g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
-          count = scan_runs<kPhasedBuildTeam, kPhasedBuildSlots>(
-              runs, n_runs, t, team_lane0, d.box, entry, accept, put, kShiftMode{});
-        } else {
-          count = scan_runs<kPhasedBuildTeam, kPhasedBuildSlots>(
-              runs, n_runs, t, team_lane0, d.box, entry, accept, put, kGenericMode{});
-        }
+        count = scan_runs<kPhasedBuildTeam, kPhasedBuildSlots>(runs, n_runs, t, team_lane0, d.box,
+                                                               entry, accept, put, kGenericMode{});
       }
       if (t == 0) {
         A.nbr_count[d.atom0 + i] = min(count, maxn);
