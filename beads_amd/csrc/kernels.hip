@@ -961,25 +961,26 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
 }
 
 // The build for systems whose atoms make too few waves at kBuildTeam lanes
-// each: kWideTeam lanes per atom, no LDS stage and no workgroup-wide phase.
-// What bounds it is one atom's serial chain (its runs' bounds, then a load per
-// round), so the team covers a row of cells in about one round and the next
-// round's candidates are in flight while this one's are tested.
-constexpr int kWideTeam = 16;
-constexpr int kWideSlots = 4;
-constexpr uint32_t kWideAtoms = kBlock / kWideTeam;
+// each: TEAM lanes per atom, no LDS stage and no workgroup-wide phase. What
+// bounds the smallest is one atom's serial chain (its runs' bounds, then a load
+// per round), so the next round's candidates are in flight while this one's are
+// tested; larger ones are bound by the candidates tested, so a round is two
+// slots a lane: with four, half of a short row's round is idle (100,000-bead
+// mixture 78 us against 65, 48,000-bead melt 66 against 58).
+constexpr int kWideSlots = 2;
 
-template <int EXCL, bool HALF>
+template <int EXCL, bool HALF, int TEAM>
 __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
   if (p.ctrl->rebuild == 0) {
     return;
   }
+  constexpr uint32_t kWideAtoms = kBlock / TEAM;
   __shared__ double red_lds[4];
   __shared__ uint2 run_lds[kWideAtoms * kMaxRuns];
-  const uint32_t t = threadIdx.x & (kWideTeam - 1);
-  const uint32_t team_lane0 = (threadIdx.x & 63u) & ~static_cast<uint32_t>(kWideTeam - 1);
-  const uint32_t q = xcd_block(blockIdx.x, gridDim.x) * kWideAtoms + threadIdx.x / kWideTeam;
-  uint2* const runs = run_lds + (threadIdx.x / kWideTeam) * kMaxRuns;
+  const uint32_t t = threadIdx.x & (TEAM - 1);
+  const uint32_t team_lane0 = (threadIdx.x & 63u) & ~static_cast<uint32_t>(TEAM - 1);
+  const uint32_t q = xcd_block(blockIdx.x, gridDim.x) * kWideAtoms + threadIdx.x / TEAM;
+  uint2* const runs = run_lds + (threadIdx.x / TEAM) * kMaxRuns;
   const bool direct = p.grid.path == 0;
   const CellGridView& g = p.grid;
   real4 xi = make_real4(0, 0, 0, 0);
@@ -992,7 +993,7 @@ __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
     } else {
       xi = p.cell_pos[q];  // the atom's position, .w its slot
       i = id_of(xi.w);
-      n_runs = team_runs<kWideTeam, true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi,
+      n_runs = team_runs<TEAM, true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi,
                                     cell_of_position(xi, p.box, g), t, team_lane0, runs);
     }
   }
@@ -1013,7 +1014,7 @@ __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
         const real4 x = p.pos[k];
         return make_real4(x.x, x.y, x.z, real_of_id(k));
       };
-      count = scan_runs<kWideTeam, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
+      count = scan_runs<TEAM, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
                                                put, kGenericMode{});
     } else {
       const char* cp_bytes = reinterpret_cast<const char*>(p.cell_pos);
@@ -1022,10 +1023,10 @@ __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
                                                k * static_cast<uint32_t>(sizeof(real4)));
       };
       if (g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
-        count = scan_runs<kWideTeam, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
+        count = scan_runs<TEAM, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
                                                  put, kShiftMode{});
       } else {
-        count = scan_runs<kWideTeam, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
+        count = scan_runs<TEAM, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
                                                  put, kGenericMode{});
       }
     }
@@ -1527,12 +1528,13 @@ void launch_pack_records(const PackParams& p, hipStream_t stream) {
   pack_records_kernel<<<grid_for(p.n), kBlock, 0, stream>>>(p);
 }
 
-// Atoms up to which the wide build is used. Measured, narrow / wide, us per
-// build (equilibrated systems): bead-spring melt of 8,000 beads 96 / 27, of
-// 27,000 101 / 46, of 64,000 108 / 73, of 100,000 140 / 104, of 216,000
-// 205 / 204, of 512,000 384 / 440; LJ fluid of 500 25 / 10, of 4,000 65 / 17,
-// of 32,000 64 / 38, of 108,000 97 / 83, of 256,000 157 / 171; four-type
-// mixture of 64,000 62 / 56, of 100,000 75 / 76, of 216,000 119 / 139.
+// Atoms up to which the wide build is used, and its 32-lane shape. Measured,
+// 4 lanes / 16 / 32, us per build (equilibrated systems): LJ fluid of 4,000
+// beads 65 / 18 / 14, of 32,000 64 / 34 / 39; bead-spring melt of 8,000
+// 96 / 24 / 21, of 48,000 106 / 58 / 67, of 100,000 140 / 100 / 122; four-type
+// mixture of 100,000 75 / 65 / 92. Above, 4 / 16 lanes with four slots: melt of
+// 216,000 205 / 204, of 512,000 384 / 440; mixture of 216,000 119 / 139.
+constexpr uint32_t kWideBuild32Max = 12000;
 constexpr uint32_t kWideBuildMax = 100000;
 
 void launch_pack_state(const PackStateParams& p, hipStream_t stream) {
@@ -1556,12 +1558,14 @@ void launch_build(const BuildParams& params, hipStream_t stream) {
   const int ex = p.spill_index != nullptr
                      ? -1
                      : (p.ecap == 0 ? 0 : (p.ecap <= 4 ? 4 : (p.ecap <= 8 ? 8 : -1)));
-  const bool wide = p.n <= kWideBuildMax;
-  const unsigned gw = grid_for(params.n, kWideAtoms);
+  const int team = p.n <= kWideBuild32Max ? 32 : (p.n <= kWideBuildMax ? 16 : kBuildTeam);
+  const unsigned gw = grid_for(params.n, kBlock / team);
 #define BEADS_BUILD_CASE(E, H)                                          \
   if (ex == E && (p.half != 0) == H) {                                  \
-    if (wide) {                                                         \
-      build_wide_kernel<E, H><<<gw, kBlock, 0, stream>>>(p);            \
+    if (team == 32) {                                                   \
+      build_wide_kernel<E, H, 32><<<gw, kBlock, 0, stream>>>(p);        \
+    } else if (team == 16) {                                            \
+      build_wide_kernel<E, H, 16><<<gw, kBlock, 0, stream>>>(p);        \
     } else {                                                            \
       build_kernel<E, H><<<g, kBlock, lds, stream>>>(p);                \
     }                                                                   \
