@@ -165,6 +165,7 @@ __global__ __launch_bounds__(kBlock) void fm_backward_kernel(AdjointParams p) {
     const double gix = gi.x, giy = gi.y, giz = gi.z;
     const real_t L0 = p.box.L[0], L1 = p.box.L[1], L2 = p.box.L[2];
     const real_t h0 = p.box.hL[0], h1 = p.box.hL[1], h2 = p.box.hL[2];
+    const real_t hmin = shortest_half(p.box);
     double gx = 0.0, gy = 0.0, gz = 0.0;
     double fx = 0.0, fy = 0.0, fz = 0.0;
     double re[TREG > 0 ? TREG : 1], rs[TREG > 0 ? TREG : 1];
@@ -191,9 +192,7 @@ __global__ __launch_bounds__(kBlock) void fm_backward_kernel(AdjointParams p) {
         real_t dx = xi.x - xj[u].x;
         real_t dy = xi.y - xj[u].y;
         real_t dz = xi.z - xj[u].z;
-        if ((__builtin_amdgcn_ballot_w64(fabs(dx) > h0) |
-             __builtin_amdgcn_ballot_w64(fabs(dy) > h1) |
-             __builtin_amdgcn_ballot_w64(fabs(dz) > h2)) != 0) {
+        if (past_half(dx, dy, dz, hmin)) {
           dx = mic_diff(xi.x, xj[u].x, L0, h0);
           dy = mic_diff(xi.y, xj[u].y, L1, h1);
           dz = mic_diff(xi.z, xj[u].z, L2, h2);

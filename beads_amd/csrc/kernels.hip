@@ -1128,6 +1128,7 @@ __device__ __forceinline__ void lj_team(const ForceParams& p, uint32_t i, uint32
   const real_t L0 = p.box.L[0], L1 = p.box.L[1], L2 = p.box.L[2];
   const real_t h0 = p.box.hL[0], h1 = p.box.hL[1], h2 = p.box.hL[2];
   const real_t xm0 = xi4.x - L0, xm1 = xi4.y - L1, xm2 = xi4.z - L2;
+  const real_t hmin = shortest_half(p.box);
   const uint32_t cnt = p.nbr_count[i];
   for (uint32_t base = 0; base < cnt; base += TEAM * SLOTS) {
     // Every slot of the round lies inside the atom's padded capacity; slots
@@ -1157,12 +1158,11 @@ __device__ __forceinline__ void lj_team(const ForceParams& p, uint32_t i, uint32
     for (int u = 0; u < SLOTS; ++u) {
       // mic_diff_sel returns the raw difference unless it exceeds half the
       // box; the folded forms are formed only when some lane of the wave
-      // needs them (pairs across a periodic boundary), the same values.
+      // may need them (pairs across a periodic boundary), the same values.
       real_t dx = xi4.x - xj[u].x;
       real_t dy = xi4.y - xj[u].y;
       real_t dz = xi4.z - xj[u].z;
-      if ((__builtin_amdgcn_ballot_w64(fabs(dx) > h0) | __builtin_amdgcn_ballot_w64(fabs(dy) > h1) |
-           __builtin_amdgcn_ballot_w64(fabs(dz) > h2)) != 0) {
+      if (past_half(dx, dy, dz, hmin)) {
         dx = mic_diff_sel(xi4.x, xm0, xj[u].x, L0, h0);
         dy = mic_diff_sel(xi4.y, xm1, xj[u].y, L1, h1);
         dz = mic_diff_sel(xi4.z, xm2, xj[u].z, L2, h2);
@@ -1363,7 +1363,7 @@ __global__ __launch_bounds__(kReduceBlock) void step_reduce_kernel(ForceParams p
 // consecutive slots of one cell, a few cache lines per atom instead of one
 // line per lane. The team's FP64 partial sums meet in a shuffle butterfly and
 // the atom's total is rounded to binary32 once.
-template <bool KICK, bool OBS, int TYPES, bool HALF, bool SPILL, int TEAM, int SLOTS>
+template <bool KICK, bool OBS, int TYPES, bool HALF, bool SPILL, bool LISTED, int TEAM, int SLOTS>
 __global__ __launch_bounds__(kBlock) void force_kernel(ForceParams p) {
   __shared__ LjCoeff lj_lds[TYPES == 1 && !HALF ? kMaxLdsTypes * kMaxLdsTypes : 1];
   __shared__ double red_lds[4];
@@ -1393,7 +1393,7 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceParams p) {
     } else {
       lj_team<OBS, TYPES, TEAM, SLOTS>(p, i, t, xi4, lj_lds, c0, fxd, fyd, fzd, sums.e_pair, sums.w_pair);
     }
-    if (p.topo.has_listed) {
+    if (LISTED && p.topo.has_listed) {
       listed_team<OBS, SPILL, TEAM>(p.pos, p.topo, p.box, p.n, i, t, xi4, fxd, fyd, fzd, sums);
     }
     fxd = team_sum<TEAM>(fxd);
@@ -1623,20 +1623,24 @@ void launch_force(const ForceParams& params, bool kick, bool obs, bool sums, hip
   const unsigned gf = grid_for(p.n, kBlock / shape.team);
 #define BEADS_FORCE_SHAPE(K, O, T, N, S)                                               \
   if (shape.team == N && shape.slots == S) {                                           \
-    force_kernel<K, O, T, false, false, N, S><<<gf, kBlock, 0, stream>>>(p);           \
+    if (p.topo.has_listed) {                                                           \
+      force_kernel<K, O, T, false, false, true, N, S><<<gf, kBlock, 0, stream>>>(p);   \
+    } else {                                                                           \
+      force_kernel<K, O, T, false, false, false, N, S><<<gf, kBlock, 0, stream>>>(p);  \
+    }                                                                                  \
   }
 #define BEADS_FORCE_CASE(K, O, T)                                                      \
   if (kick == K && obs == O && (half || types == T)) {                                 \
     if (half) {                                                                        \
       if (spill) {                                                                     \
-        force_kernel<K, O, 0, true, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);         \
+        force_kernel<K, O, 0, true, true, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);         \
       } else {                                                                         \
-        force_kernel<K, O, 0, true, false, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
+        force_kernel<K, O, 0, true, false, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
       }                                                                                \
       if (sums) step_reduce_kernel<K, O, true><<<1, kReduceBlock, 0, stream>>>(p, gf); \
     } else {                                                                           \
       if (spill) {                                                                     \
-        force_kernel<K, O, T, false, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
+        force_kernel<K, O, T, false, true, true, 4, 8><<<gf, kBlock, 0, stream>>>(p);        \
       } else {                                                                         \
         BEADS_FORCE_SHAPE(K, O, T, 4, 8)                                               \
         BEADS_FORCE_SHAPE(K, O, T, 8, 4)                                               \

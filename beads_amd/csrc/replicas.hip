@@ -310,6 +310,7 @@ __device__ __forceinline__ void force_atom(const ReplicaDesc& d, const real4* po
   const uint32_t n = d.n;
   const real_t L0 = d.box.L[0], L1 = d.box.L[1], L2 = d.box.L[2];
   const real_t h0 = d.box.hL[0], h1 = d.box.hL[1], h2 = d.box.hL[2];
+  const real_t hmin = shortest_half(d.box);
   const int T = d.n_types;
   const LjCoeff c0 = lj[0];
   const real4 xi = pos[i];
@@ -335,8 +336,7 @@ __device__ __forceinline__ void force_atom(const ReplicaDesc& d, const real4* po
       real_t dx = xi.x - xj[u].x;
       real_t dy = xi.y - xj[u].y;
       real_t dz = xi.z - xj[u].z;
-      if ((__builtin_amdgcn_ballot_w64(fabs(dx) > h0) | __builtin_amdgcn_ballot_w64(fabs(dy) > h1) |
-           __builtin_amdgcn_ballot_w64(fabs(dz) > h2)) != 0) {
+      if (past_half(dx, dy, dz, hmin)) {
         dx = mic_diff(xi.x, xj[u].x, L0, h0);
         dy = mic_diff(xi.y, xj[u].y, L1, h1);
         dz = mic_diff(xi.z, xj[u].z, L2, h2);
