@@ -99,6 +99,16 @@ __global__ __launch_bounds__(kBlock) void pack_xyz_kernel(uint32_t n, const real
   out[i] = make_real4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], 0);
 }
 
+// Positions and dL/dF interleaved, so that a partner's two records share a
+// cache line.
+__global__ __launch_bounds__(kBlock) void pack_frame_kernel(uint32_t n, const real4* pos,
+                                                            const real_t* xyz, real4* out) {
+  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n) return;
+  out[2 * i] = pos[i];
+  out[2 * i + 1] = make_real4(xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], 0);
+}
+
 // Lanes per atom and list slots per lane per round of the backward pass (the
 // force pass's team layout: lane t takes slots base + u*kAdjTeam + t).
 constexpr int kAdjTeam = 4;
@@ -140,8 +150,12 @@ __device__ __forceinline__ AdjLj adj_lj(const AdjointParams& p, int k) {
 // One type: the pair factors live in registers; more: in an LDS table.
 // GE: dL/dE is nonzero, so the pass also sums F for the -gE F term and the
 // energy's parameter derivatives. Each atom's team sums its partial dL/dx in
-// FP64 before the store.
-template <int TREG, bool GE>
+// FP64 before the store. STRIDE: records from one atom to the next in p.pos and
+// p.g: 2 when they are interleaved (pack_frame_kernel), 1 when apart. The pass
+// is bound by its gathers, most of all in a caller's order, where every partner
+// is a cache line of its own in each array: 110 us apart and 86
+// interleaved at 100,000 shuffled beads of four types.
+template <int TREG, bool GE, int STRIDE>
 __global__ __launch_bounds__(kBlock) void fm_backward_kernel(AdjointParams p) {
   __shared__ double acc[2 * kMaxLdsTypes * kMaxLdsTypes + 2 * kMaxBondTypesAdjoint];
   __shared__ AdjLj coef[TREG == 1 ? 1 : kMaxLdsTypes * kMaxLdsTypes];
@@ -159,9 +173,9 @@ __global__ __launch_bounds__(kBlock) void fm_backward_kernel(AdjointParams p) {
   const uint32_t i = xcd_block(blockIdx.x, gridDim.x) * kAdjAtoms + threadIdx.x / kAdjTeam;
   const double gE = p.grad_energy;
   if (i < n) {  // uniform over a team
-    const real4 xi = p.pos[i];
+    const real4 xi = p.pos[STRIDE * i];
     const int ti = static_cast<int>(id_of(xi.w));
-    const real4 gi = p.g[i];
+    const real4 gi = p.g[STRIDE * i];
     const double gix = gi.x, giy = gi.y, giz = gi.z;
     const real_t L0 = p.box.L[0], L1 = p.box.L[1], L2 = p.box.L[2];
     const real_t h0 = p.box.hL[0], h1 = p.box.hL[1], h2 = p.box.hL[2];
@@ -182,8 +196,8 @@ __global__ __launch_bounds__(kBlock) void fm_backward_kernel(AdjointParams p) {
       real4 xj[kAdjSlots], gj[kAdjSlots];
 #pragma unroll
       for (int u = 0; u < kAdjSlots; ++u) {
-        xj[u] = p.pos[jj[u]];
-        gj[u] = p.g[jj[u]];
+        xj[u] = p.pos[STRIDE * jj[u]];
+        gj[u] = p.g[STRIDE * jj[u]];
       }
 #pragma unroll
       for (int u = 0; u < kAdjSlots; ++u) {
@@ -265,14 +279,14 @@ __global__ __launch_bounds__(kBlock) void fm_backward_kernel(AdjointParams p) {
                                          : p.spill_bond[spill_off + (k - nbond_inline)];
         const uint32_t bt = r.y & 0x7fffffffu;
         const double kk = p.bond_k[bt], r0 = p.bond_r0[bt];
-        const real3 d = mic3(x3, f3(p.pos[r.x]), p.box);
+        const real3 d = mic3(x3, f3(p.pos[STRIDE * r.x]), p.box);
         const double ddx = d.x, ddy = d.y, ddz = d.z;
         const double rr = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
         if (rr == 0.0) continue;
         const double inv_r = rcp_f64(rr);
         const double phi = -kk * (rr - r0) * inv_r;
         const double dphi_r = -kk * r0 * inv_r * inv_r * inv_r;  // phi' / r
-        const real4 gp = p.g[r.x];
+        const real4 gp = p.g[STRIDE * r.x];
         const double ex = gix - gp.x, ey = giy - gp.y, ez = giz - gp.z;
         const double dd = ddx * ex + ddy * ey + ddz * ez;
         gx += phi * ex + dphi_r * ddx * dd;
@@ -478,6 +492,7 @@ __device__ RoleAdjoint dihedral_adjoint(real3 q0, real3 q1, real3 q2, real3 q3, 
 constexpr int kListTeam = 4;
 constexpr uint32_t kListAtoms = kBlock / kListTeam;
 
+template <int STRIDE>
 __global__ __launch_bounds__(kBlock) void listed_backward_kernel(AdjointParams p) {
   __shared__ double acc[2 * kMaxAngleTypesAdjoint + kMaxDihedralTypesAdjoint];
   const int na = p.n_angle_types, nd = p.n_dihedral_types;
@@ -489,8 +504,8 @@ __global__ __launch_bounds__(kBlock) void listed_backward_kernel(AdjointParams p
   const uint32_t i = blockIdx.x * kListAtoms + threadIdx.x / kListTeam;
   const double gE = p.grad_energy;
   if (i < n) {  // uniform over a team
-    const real3 xi = f3(p.pos[i]);
-    const real4 gi = p.g[i];
+    const real3 xi = f3(p.pos[STRIDE * i]);
+    const real4 gi = p.g[STRIDE * i];
     const uint32_t cw = p.topo_count[i];
     const uint32_t ang_inline = p.acap > 0 ? (cw >> 8) & 255u : 0u;
     const uint32_t dih_inline = p.dcap > 0 ? (cw >> 16) & 255u : 0u;
@@ -517,8 +532,8 @@ __global__ __launch_bounds__(kBlock) void listed_backward_kernel(AdjointParams p
       const uint4 r = k < ang_inline ? p.angle[static_cast<size_t>(k) * n + i]
                                      : p.spill_angle[off_a + (k - ang_inline)];
       const int role = static_cast<int>(r.w);
-      const real3 a = f3(p.pos[r.x]), b = f3(p.pos[r.y]);
-      const real4 ga = p.g[r.x], gb = p.g[r.y];
+      const real3 a = f3(p.pos[STRIDE * r.x]), b = f3(p.pos[STRIDE * r.y]);
+      const real4 ga = p.g[STRIDE * r.x], gb = p.g[STRIDE * r.y];
       const real3 pi = role == 0 ? xi : a;
       const real3 pj = role == 0 ? a : (role == 1 ? xi : b);
       const real3 pk = role == 2 ? xi : b;
@@ -536,8 +551,8 @@ __global__ __launch_bounds__(kBlock) void listed_backward_kernel(AdjointParams p
                                      : p.spill_dih[off_d + (k - dih_inline)];
       const int role = static_cast<int>(r.w >> 30);
       const uint32_t ty = r.w & 0x3fffffffu;
-      const real3 a = f3(p.pos[r.x]), b = f3(p.pos[r.y]), c = f3(p.pos[r.z]);
-      const real4 ga = p.g[r.x], gb = p.g[r.y], gc = p.g[r.z];
+      const real3 a = f3(p.pos[STRIDE * r.x]), b = f3(p.pos[STRIDE * r.y]), c = f3(p.pos[STRIDE * r.z]);
+      const real4 ga = p.g[STRIDE * r.x], gb = p.g[STRIDE * r.y], gc = p.g[STRIDE * r.z];
       real3 q0, q1, q2, q3;
       real4 h0, h1, h2, h3;
       if (role == 0) { q0 = xi; q1 = a; q2 = b; q3 = c; h0 = gi; h1 = ga; h2 = gb; h3 = gc; }
@@ -611,22 +626,37 @@ void launch_pack_xyz(uint32_t n, const real_t* xyz, real4* out, hipStream_t stre
   pack_xyz_kernel<<<grid_for(n), kBlock, 0, stream>>>(n, xyz, out);
 }
 
-void launch_fm_backward(const AdjointParams& p, hipStream_t stream) {
+void launch_pack_frame(uint32_t n, const real4* pos, const real_t* xyz, real4* out,
+                       hipStream_t stream) {
+  pack_frame_kernel<<<grid_for(n), kBlock, 0, stream>>>(n, pos, xyz, out);
+}
+
+namespace {
+
+template <int STRIDE>
+void launch_backward(const AdjointParams& p, hipStream_t stream) {
   const unsigned g = grid_for(p.n, kAdjAtoms);
   const bool ge = p.grad_energy != 0.0;
   if (p.n_types <= 1) {
-    if (ge) fm_backward_kernel<1, true><<<g, kBlock, 0, stream>>>(p);
-    else fm_backward_kernel<1, false><<<g, kBlock, 0, stream>>>(p);
+    if (ge) fm_backward_kernel<1, true, STRIDE><<<g, kBlock, 0, stream>>>(p);
+    else fm_backward_kernel<1, false, STRIDE><<<g, kBlock, 0, stream>>>(p);
   } else if (p.n_types <= 4) {
-    if (ge) fm_backward_kernel<4, true><<<g, kBlock, 0, stream>>>(p);
-    else fm_backward_kernel<4, false><<<g, kBlock, 0, stream>>>(p);
+    if (ge) fm_backward_kernel<4, true, STRIDE><<<g, kBlock, 0, stream>>>(p);
+    else fm_backward_kernel<4, false, STRIDE><<<g, kBlock, 0, stream>>>(p);
   } else {
-    if (ge) fm_backward_kernel<0, true><<<g, kBlock, 0, stream>>>(p);
-    else fm_backward_kernel<0, false><<<g, kBlock, 0, stream>>>(p);
+    if (ge) fm_backward_kernel<0, true, STRIDE><<<g, kBlock, 0, stream>>>(p);
+    else fm_backward_kernel<0, false, STRIDE><<<g, kBlock, 0, stream>>>(p);
   }
   if (p.acap > 0 || p.dcap > 0) {
-    listed_backward_kernel<<<grid_for(p.n, kListAtoms), kBlock, 0, stream>>>(p);
+    listed_backward_kernel<STRIDE><<<grid_for(p.n, kListAtoms), kBlock, 0, stream>>>(p);
   }
+}
+
+}  // namespace
+
+void launch_fm_backward(const AdjointParams& p, bool interleaved, hipStream_t stream) {
+  if (interleaved) launch_backward<2>(p, stream);
+  else launch_backward<1>(p, stream);
 }
 
 }  // namespace beads_amd

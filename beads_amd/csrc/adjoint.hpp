@@ -19,8 +19,10 @@ constexpr uint32_t kNoAllocMaxAtoms = 1u << 20;
 
 struct AdjointParams {
   uint32_t n;
-  const real4* pos;        // positions, .w = type bits
-  const real4* g;          // dL/dF per atom
+  // Positions (.w = type bits) and dL/dF per atom: arrays apart, or interleaved
+  // records {pos, g} (launch_fm_backward's argument).
+  const real4* pos;
+  const real4* g;
   const uint32_t* nbr_count;
   const uint32_t* nbr;      // chunked full list
   BoxView box;
@@ -78,11 +80,14 @@ struct FrameLoadParams {
 void launch_frame_load(const FrameLoadParams& p, bool check, hipStream_t stream);
 void launch_frame_store(uint32_t n, const real4* force, real_t* xyz, hipStream_t stream);
 void launch_pack_xyz(uint32_t n, const real_t* xyz, real4* out, hipStream_t stream);
+// out[2 i] = pos[i], out[2 i + 1] = xyz of atom i.
+void launch_pack_frame(uint32_t n, const real4* pos, const real_t* xyz, real4* out,
+                       hipStream_t stream);
 // out[0, count) = 0 with a kernel (no memset node when a caller captures the stream).
 void launch_fill_f64(double* out, uint32_t count, hipStream_t stream);
 // This GPU's static staging array (kNoAllocMaxAtoms real4), address resolved
 // once per device; allocates nothing.
 real4* scratch_address();
-void launch_fm_backward(const AdjointParams& p, hipStream_t stream);
+void launch_fm_backward(const AdjointParams& p, bool interleaved, hipStream_t stream);
 
 }  // namespace beads_amd

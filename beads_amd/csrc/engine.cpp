@@ -1198,7 +1198,7 @@ void Engine::frame_backward(const real_t* grad_forces_dev, double grad_energy,
     staging = scratch_address();
     async = true;
   } else {
-    grad_force4_.resize(n_);
+    grad_force4_.resize(2 * static_cast<size_t>(n_));  // interleaved with the positions
     staging = grad_force4_.data();
   }
   if (noalloc) {
@@ -1208,10 +1208,16 @@ void Engine::frame_backward(const real_t* grad_forces_dev, double grad_energy,
     BEADS_HIP(hipEventRecord(frame_events_[2], stream_));
     BEADS_HIP(hipMemsetAsync(grad_params_dev, 0, n_params * sizeof(double), stream_));
   }
-  launch_pack_xyz(n_, grad_forces_dev, staging, stream_);
   p.n = n_;
-  p.pos = pos_.data();
-  p.g = staging;
+  if (noalloc) {  // its static scratch holds dL/dF alone
+    launch_pack_xyz(n_, grad_forces_dev, staging, stream_);
+    p.pos = pos_.data();
+    p.g = staging;
+  } else {
+    launch_pack_frame(n_, pos_.data(), grad_forces_dev, staging, stream_);
+    p.pos = staging;
+    p.g = staging + 1;
+  }
   p.nbr_count = nbr_count_.data();
   p.nbr = nbr_.data();
   p.box = box_;
@@ -1230,7 +1236,7 @@ void Engine::frame_backward(const real_t* grad_forces_dev, double grad_energy,
   p.grad_energy = grad_energy;
   p.grad_pos = grad_positions_dev;
   p.grad_params = grad_params_dev;
-  launch_fm_backward(p, stream_);
+  launch_fm_backward(p, !noalloc, stream_);
   BEADS_HIP(hipGetLastError());
   if (noalloc) return;
   BEADS_HIP(hipEventRecord(frame_events_[3], stream_));
