@@ -5,12 +5,13 @@
 // streams (float4, or double4 in the BEADS_REAL64 build), FP64 for LJ pair
 // values and global reductions. Kernels that gather
 // neighbour positions map workgroups onto atoms XCD by XCD so each XCD's L2
-// holds one contiguous (spatially sorted) slab of positions. Every kernel of
-// the neighbour-rebuild sequence reads the device control block first and
-// exits when no rebuild is due, so a step never waits on the host. No kernel
-// fences at device scope (on gfx950 that is an L2 write-back and invalidate
-// of the XCD): cross-workgroup totals are formed by a one-workgroup kernel
-// launched after the workgroups that wrote the partials.
+// holds one contiguous (spatially sorted) slab of positions. The two kernels of
+// the neighbour-rebuild sequence read the device control block first and exit
+// when no rebuild is due, so a step never waits on the host. No kernel that runs
+// every step fences at device scope (on gfx950 that is an L2 write-back and
+// invalidate of the XCD): cross-workgroup totals are formed by a one-workgroup
+// kernel launched after the workgroups that wrote the partials. Only a reorder,
+// inside the rebuild kernel, hands bulk data between workgroups with one.
 //
 // Reference counterparts (paths under native/src):
 //   control/bin/scan/scatter/sort  simulation/neighbor/cell_list_build.cu:110-219,347-414,
