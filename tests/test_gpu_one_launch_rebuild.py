@@ -61,3 +61,31 @@ def test_cells_of_more_than_a_wave():
     w = _every_step(W.lj_box(6000, 0.8, 1.0, seed=4, cutoff=5.0)).with_(max_neighbors=768)
     assert w.n / O.plan(w).n_cells > 64
     _final_state(w, 10)
+
+
+def test_engines_rebuilding_side_by_side():
+    """Several engines step on their own streams at once, each rebuilding every
+    step: whichever workgroups of a rebuild the GPU holds, the result is that of
+    the engine alone."""
+    ws = [_every_step(W.lj_box(n, 0.8, 1.0, seed=n)) for n in (3000, 40000, 20000, 60000)]
+    alone = []
+    for w in ws:
+        with Engine(w) as e:
+            e.initialize(observables=False)
+            e.advance(48)
+            alone.append(e.state())
+    engines = [Engine(w) for w in ws]
+    try:
+        for e in engines:
+            e.initialize(observables=False)
+        for _ in range(3):  # calls return at once, so the engines' steps overlap
+            for e in engines:
+                e.advance(16)
+        for e, a in zip(engines, alone):
+            s = e.state()
+            assert e.stats().overflow == 0
+            for k in ("positions", "velocities", "tags", "images"):
+                assert np.array_equal(s[k], a[k]), k
+    finally:
+        for e in engines:
+            e.close()
