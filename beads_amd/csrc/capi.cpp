@@ -272,6 +272,26 @@ beads_status_t beads_engine_frame_backward_noalloc(beads_engine_t* e, const bead
   });
 }
 
+// Not part of the API (undeclared in beads_amd.h): what tests need to force a
+// rebuild that only some workgroups share, or one that stalls.
+beads_status_t beads_internal_rebuild_limits(beads_engine_t* e, uint32_t members,
+                                             int64_t join_ticks, uint32_t wait_polls) {
+  return guarded([&] {
+    beads_amd::RebuildLimits limits;
+    limits.members = members;
+    limits.join_ticks = join_ticks;
+    limits.wait_polls = wait_polls;
+    engine_of(e).set_rebuild_limits(limits);
+  });
+}
+
+beads_status_t beads_internal_rebuild_members(beads_engine_t* e, uint32_t* members) {
+  return guarded([&] {
+    beads_amd::require(members != nullptr, "members output is null");
+    *members = engine_of(e).rebuild_members();
+  });
+}
+
 void beads_engine_destroy(beads_engine_t* e) {
   if (e != nullptr) {
     delete e->impl;

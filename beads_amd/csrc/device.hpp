@@ -74,9 +74,6 @@ struct CellGridView {
 constexpr uint32_t kNeighborParts = 64;
 constexpr uint32_t kNeighborPartStride = 16;
 
-// Ctrl::overflow when a wait between a rebuild's workgroups passed its bound.
-constexpr uint32_t kRebuildStalled = 2;
-
 // Device-resident control block. Written only by kernels (and zeroed once at
 // set-up), read back asynchronously by the host.
 struct alignas(256) Ctrl {
@@ -84,7 +81,10 @@ struct alignas(256) Ctrl {
   uint32_t reorder;         // the rebuild also sorts particles into cell order
   uint32_t joined;          // workgroups that joined this step's rebuild (rebuild_kernel)
   uint32_t checked;         // a scheduled check ran since the last build
-  uint32_t overflow;        // 1: a neighbour list overflowed; kRebuildStalled
+  uint32_t overflow;        // a neighbour list overflowed
+  uint32_t stalled;         // a wait inside a rebuild passed its bound: no rebuild or
+                            // build does anything any more (rebuild_kernel)
+  uint32_t members;         // workgroups that shared the last rebuild
   uint64_t build_count;
   uint64_t dangerous;
   uint64_t reorder_count;

@@ -612,6 +612,8 @@ void Engine::upload_state() {
   sync_lines_.resize(2 * kRebuildMaxBlocks * kSyncLine);
   sync_lines_.zero(stream_);
   tile_sums_.resize(kRebuildMaxBlocks);
+  stalled_host_.resize(1);
+  *stalled_host_.data() = 0;
   Ctrl c{};
   c.lambda = 1.0;
   ctrl_.upload(&c, 1, stream_);
@@ -734,6 +736,7 @@ void Engine::set_up_params() {
   rb.neighbor_parts = neighbor_parts_.data();
   rb.sync_lines = sync_lines_.data();
   rb.tile_sums = tile_sums_.data();
+  rb.stalled_host = stalled_host_.data();
 
   ReorderParams& r = reorder_params_;
   r.n = n_;
@@ -806,6 +809,7 @@ void Engine::force_pass(bool kick, bool observables, bool sums) {
 
 void Engine::initialize(bool observables) {
   require(!frame_mode_, "an engine used in frame mode cannot run dynamics.", BEADS_E_RUNTIME);
+  check_rebuilds();
   rebuild_sequence(true, 0);
   force_pass(false, observables);
   BEADS_HIP(hipGetLastError());
@@ -862,6 +866,7 @@ void Engine::replay_step_graph() {
 
 void Engine::advance(uint64_t n_steps, bool observables_on_last) {
   require(initialized_, "engine must be initialized before advancing.", BEADS_E_RUNTIME);
+  check_rebuilds();
   const uint64_t g = graph_steps();
   uint64_t left = n_steps;
   while (left > 0) {
@@ -887,6 +892,7 @@ void Engine::materialize_velocities() {
 // overflow that async frame calls left unchecked.
 void Engine::synchronize() {
   BEADS_HIP(hipStreamSynchronize(stream_));
+  check_rebuilds();
   if (frame_mode_) check_overflow(fetch_ctrl());
 }
 
@@ -894,12 +900,32 @@ Ctrl Engine::fetch_ctrl() {
   BEADS_HIP(hipMemcpyAsync(ctrl_host_.data(), ctrl_.data(), sizeof(Ctrl), hipMemcpyDeviceToHost,
                            stream_));
   BEADS_HIP(hipStreamSynchronize(stream_));
+  check_rebuilds();
   return *ctrl_host_.data();
 }
 
+// Reports a rebuild that stalled in the work that has completed so far; the
+// engine's state is lost with it.
+void Engine::check_rebuilds() const {
+  const volatile uint32_t* const stalled = stalled_host_.data();
+  require(*stalled == 0, "the neighbor rebuild's workgroups lost each other.", BEADS_E_DEVICE);
+}
+
+void Engine::set_rebuild_limits(const RebuildLimits& limits) {
+  require(limits.members > 0 && limits.members <= kRebuildMaxBlocks && limits.join_ticks >= 0,
+          "rebuild limits are out of range.");
+  BEADS_HIP(hipStreamSynchronize(stream_));
+  rebuild_params_.limits = limits;
+  if (step_graph_exec_ != nullptr) {  // holds the limits it was captured with
+    BEADS_HIP(hipGraphExecDestroy(step_graph_exec_));
+    step_graph_exec_ = nullptr;
+  }
+}
+
+uint32_t Engine::rebuild_members() { return fetch_ctrl().members; }
+
 void Engine::check_overflow(const Ctrl& c) {
-  require(c.overflow != kRebuildStalled, "the neighbor rebuild's workgroups lost each other.",
-          BEADS_E_DEVICE);
+  check_rebuilds();
   if (c.overflow != 0) {
     std::ostringstream m;
     m << "NeighborList overflow"
@@ -956,6 +982,7 @@ void Engine::read_state(const beads_state_out_t& o) {
   src.tag = tag_.data();
   src.molid = molid_.data();
   state_reader_.read(src, o, stream_);
+  check_rebuilds();
   if (frame_mode_) check_overflow(fetch_ctrl());
 }
 

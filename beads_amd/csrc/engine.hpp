@@ -128,6 +128,10 @@ class Engine {
   void frame_timing(double* forward_s, double* backward_s);
   // Enqueue frame-mode work on the caller's stream (nullptr: the engine's own).
   void set_stream(hipStream_t stream);
+  // How the workgroups of a rebuild meet, for tests that force a partial or a
+  // stalled one, and how many shared the last rebuild.
+  void set_rebuild_limits(const RebuildLimits& limits);
+  uint32_t rebuild_members();
   uint32_t n_particles() const { return n_; }
   int32_t n_types() const { return n_types_; }
   int32_t n_bond_types() const { return n_bond_types_; }
@@ -146,6 +150,7 @@ class Engine {
   uint64_t graph_steps() const;
   void replay_step_graph();
   void materialize_velocities();
+  void check_rebuilds() const;
   Ctrl fetch_ctrl();
   void check_overflow(const Ctrl& c);
   bool output_due(uint64_t step) const;
@@ -209,6 +214,7 @@ class Engine {
   DeviceBuffer<unsigned long long> neighbor_parts_;
   DeviceBuffer<uint64_t> sync_lines_;  // rebuild_kernel's meeting points
   DeviceBuffer<uint32_t> tile_sums_;
+  PinnedBuffer<uint32_t> stalled_host_;  // nonzero: a rebuild stalled
   PinnedBuffer<Ctrl> ctrl_host_;
   uint32_t bcap_ = 0, acap_ = 0, dcap_ = 0, ecap_ = 0;
   bool has_topology_ = false;

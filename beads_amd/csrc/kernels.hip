@@ -99,10 +99,19 @@ __global__ __launch_bounds__(kNeighborParts) void control_kernel(
 //
 // Which workgroups take part is settled at run time, so that no wait depends
 // on how many of them the GPU holds at once: a workgroup that starts joins by
-// taking a rank; rank 0 closes the list when all have joined, or kJoinTicks
+// taking a rank; rank 0 closes the list when all have joined, or join_ticks
 // after its own start, and a workgroup that starts later leaves at once. The
 // members are all running when the list closes and wait only for each other,
 // so every wait ends. Work is divided by rank over the members there are.
+//
+// Every wait is bounded all the same (wait_polls). Past the bound a member
+// stores Ctrl::stalled and leaves, which fails the others' next barrier; up to
+// it each phase has read only what the barriers before it completed. From then
+// on the cells, and a reorder's arrays, may be half done, so the state is
+// final: no later launch bins, sorts or builds (counts that were not cleared
+// would run the scatter past its array), the force pass keeps the last whole
+// list, whose slots stay inside every array, and every host call that
+// waits for the engine reports the stall.
 //
 // Each member has a cache line of its own to arrive on and one to be released
 // on: polls and stores of 256 workgroups on one word would serialise (33 ns
@@ -113,13 +122,10 @@ constexpr uint32_t kJoinClosed = 0x80000000u;
 constexpr uint32_t kRankBits = 9;  // ranks and counts up to kRebuildMaxBlocks
 static_assert(kRebuildMaxBlocks < (1u << kRankBits) && kRebuildMaxBlocks <= kRebuildBlock,
               "rank 0 polls one member per thread");
-// wall_clock64 ticks (100 MHz): how long rank 0 waits for the grid to start,
-// and the bound on any other wait, which only a fault can reach.
-constexpr long long kJoinTicks = 3000;
-constexpr long long kWaitTicks = 400000000;
-
 struct Members {
   uint64_t* lines;  // [member][2 * kSyncLine]: arrival word, release word a line later
+  uint32_t* stalled_host;
+  uint32_t wait_polls;
   uint32_t rank, count;
   uint64_t epoch;   // unique to this rebuild and barrier, advanced by each barrier
 };
@@ -134,38 +140,53 @@ __device__ __forceinline__ void agent_store(T* p, T v) {
 }
 
 // Waits until *word holds the epoch above its kRankBits; false past the bound.
-__device__ __forceinline__ bool await_epoch(const uint64_t* word, uint64_t epoch) {
-  const long long start = wall_clock64();
-  while ((agent_load(word) >> kRankBits) != epoch) {
-    if (wall_clock64() - start > kWaitTicks) return false;
+__device__ __forceinline__ bool await_epoch(const uint64_t* word, const Members& m) {
+  for (uint32_t polls = 0; (agent_load(word) >> kRankBits) != m.epoch; ++polls) {
+    if (polls >= m.wait_polls) return false;
     __builtin_amdgcn_s_sleep(1);
   }
   return true;
 }
 
+__device__ __forceinline__ void report_stall(Ctrl* ctrl, const Members& m) {
+  agent_store(&ctrl->stalled, 1u);
+  __hip_atomic_store(m.stalled_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Joins the rebuild's members. Returns false (in every thread) where the
 // workgroup has nothing to do. epoch0 is above 0, which the lines start with.
-__device__ __forceinline__ bool join_members(Ctrl* ctrl, uint64_t* lines, uint64_t epoch0,
+__device__ __forceinline__ bool join_members(Ctrl* ctrl, const RebuildParams& p, uint64_t epoch0,
                                              Members& m) {
   __shared__ uint32_t rank_lds, count_lds;
+  const RebuildLimits& limits = p.limits;
+  uint64_t* const lines = p.sync_lines;
   if (threadIdx.x == 0) {
-    const uint32_t v = __hip_atomic_fetch_add(&ctrl->joined, 1u, __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
+    // Nobody joins after a stall (looked at by one thread: a stall in this very
+    // launch may come between the looks of two).
+    const uint32_t v = agent_load(&ctrl->stalled) != 0
+                           ? kJoinClosed
+                           : __hip_atomic_fetch_add(&ctrl->joined, 1u, __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
     rank_lds = v;
     count_lds = 0;
     if (v == 0) {
+      const uint32_t all = min(static_cast<uint32_t>(gridDim.x), limits.members);
       const long long start = wall_clock64();
-      while (agent_load(&ctrl->joined) < gridDim.x && wall_clock64() - start < kJoinTicks) {
+      while (agent_load(&ctrl->joined) < all && wall_clock64() - start < limits.join_ticks) {
         __builtin_amdgcn_s_sleep(1);
       }
-      count_lds = __hip_atomic_fetch_or(&ctrl->joined, kJoinClosed, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
+      count_lds = min(__hip_atomic_fetch_or(&ctrl->joined, kJoinClosed, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT),
+                      limits.members);
+      agent_store(&ctrl->members, count_lds);
     }
   }
   __syncthreads();
   const uint32_t rank = rank_lds;
-  if (rank & kJoinClosed) return false;
+  if (rank >= limits.members) return false;  // closed (kJoinClosed) or full
   m.lines = lines;
+  m.stalled_host = p.stalled_host;
+  m.wait_polls = limits.wait_polls;
   m.rank = rank;
   m.epoch = epoch0;
   if (rank == 0) {
@@ -175,10 +196,10 @@ __device__ __forceinline__ bool join_members(Ctrl* ctrl, uint64_t* lines, uint64
     }
   } else if (threadIdx.x == 0) {
     const uint64_t* const release = lines + (2 * rank + 1) * kSyncLine;
-    if (await_epoch(release, epoch0)) {
+    if (await_epoch(release, m)) {
       count_lds = static_cast<uint32_t>(agent_load(release)) & ((1u << kRankBits) - 1u);
     } else {
-      agent_store(&ctrl->overflow, kRebuildStalled);
+      report_stall(ctrl, m);
     }
   }
   __syncthreads();
@@ -206,7 +227,7 @@ __device__ __forceinline__ bool member_barrier(Ctrl* ctrl, Members& m) {
   }
   if (m.rank == 0) {
     if (threadIdx.x > 0 && threadIdx.x < m.count &&
-        !await_epoch(m.lines + 2 * threadIdx.x * kSyncLine, m.epoch)) {
+        !await_epoch(m.lines + 2 * threadIdx.x * kSyncLine, m)) {
       ok_lds = 0;
     }
     __syncthreads();
@@ -214,12 +235,12 @@ __device__ __forceinline__ bool member_barrier(Ctrl* ctrl, Members& m) {
       agent_store(m.lines + (2 * threadIdx.x + 1) * kSyncLine, m.epoch << kRankBits);
     }
   } else if (threadIdx.x == 0 &&
-             !await_epoch(m.lines + (2 * m.rank + 1) * kSyncLine, m.epoch)) {
+             !await_epoch(m.lines + (2 * m.rank + 1) * kSyncLine, m)) {
     ok_lds = 0;
   }
   __syncthreads();
   const bool ok = ok_lds != 0;
-  if (!ok && threadIdx.x == 0) agent_store(&ctrl->overflow, kRebuildStalled);
+  if (!ok && threadIdx.x == 0) report_stall(ctrl, m);
   // One wave's acquire empties the caches the workgroup reads through.
   if (FULL && threadIdx.x < 64) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   __syncthreads();
@@ -600,7 +621,9 @@ __global__ __launch_bounds__(kRebuildBlock) void rebuild_kernel(CellScanParams c
   }
   const bool reorder = reorder_due(ctrl, p.control, p.steps);
   Members m;
-  if (!join_members(ctrl, p.sync_lines, (ctrl->build_count + 1) * 8u, m)) return;
+  // The epochs of a rebuild differ from those of every other one: each whole
+  // one counts a build, and none follows one that stalled.
+  if (!join_members(ctrl, p, (ctrl->build_count + 1) * 8u, m)) return;
   const uint32_t n = cp.n;
   const uint32_t first = m.rank * kRebuildBlock + threadIdx.x;
   const uint32_t stride = m.count * kRebuildBlock;
@@ -767,7 +790,7 @@ __device__ __forceinline__ void publish_build(const BuildParams& p, uint32_t sto
 // stored once.
 template <int EXCL, bool HALF>
 __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
-  if (p.ctrl->rebuild == 0) {
+  if (p.ctrl->rebuild == 0 || p.ctrl->stalled != 0) {
     return;
   }
   __shared__ double red_lds[4];
@@ -972,7 +995,7 @@ constexpr int kWideSlots = 2;
 
 template <int EXCL, bool HALF, int TEAM>
 __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
-  if (p.ctrl->rebuild == 0) {
+  if (p.ctrl->rebuild == 0 || p.ctrl->stalled != 0) {
     return;
   }
   constexpr uint32_t kWideAtoms = kBlock / TEAM;

@@ -27,6 +27,18 @@ struct CellScanParams {
 // The rebuild kernel's bookkeeping and the memory its workgroups meet in.
 constexpr uint32_t kRebuildMaxBlocks = 256;
 constexpr uint32_t kSyncLine = 16;  // 8-byte words of a member's arrival or release line
+
+// How a rebuild's workgroups meet (rebuild_kernel).
+struct RebuildLimits {
+  uint32_t members = kRebuildMaxBlocks;  // most that take part
+  int64_t join_ticks = 3000;             // how long the first waits for the grid to start,
+                                         // in wall_clock64 ticks (100 MHz)
+  // Polls before any other wait is given up: at about a microsecond each over
+  // 4 s of running. Polls and not time, which passes for a workgroup whose
+  // queue is off the GPU too.
+  uint32_t wait_polls = 1u << 22;
+};
+
 struct RebuildParams {
   Ctrl* ctrl;
   NeighborControl control;
@@ -35,6 +47,8 @@ struct RebuildParams {
   unsigned long long* neighbor_parts;  // cleared for the build
   uint64_t* sync_lines;                // [kRebuildMaxBlocks][2 * kSyncLine], zero at set-up
   uint32_t* tile_sums;                 // [kRebuildMaxBlocks]
+  RebuildLimits limits;
+  uint32_t* stalled_host;              // host memory: Ctrl::stalled for the host to look at
 };
 
 struct ScaleParams {

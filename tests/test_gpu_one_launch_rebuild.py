@@ -10,12 +10,14 @@ neighbour sets are held bit for bit to the oracle's at the final positions.
 
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle as O
 from beads_amd import workloads as W
-from beads_amd.capi import Engine
+from beads_amd.capi import BeadsError, Engine
 
 pytestmark = pytest.mark.gpu
 
@@ -40,6 +42,18 @@ def _final_state(w, steps):
     np.testing.assert_array_equal(counts, rc)
     for i in range(0, w.n, max(1, w.n // 3000)):
         assert np.array_equal(np.sort(lst[:counts[i], i]), np.sort(rl[i, :rc[i]])), i
+
+
+def _limit(e, members=256, join_ticks=3000, wait_polls=1 << 22):
+    """How the workgroups of e's rebuilds meet from here on."""
+    e._check(e.lib.beads_internal_rebuild_limits(e.handle, C.c_uint32(members),
+                                                 C.c_int64(join_ticks), C.c_uint32(wait_polls)))
+
+
+def _members(e):
+    n = C.c_uint32()
+    e._check(e.lib.beads_internal_rebuild_members(e.handle, C.byref(n)))
+    return n.value
 
 
 def _every_step(w):
@@ -89,3 +103,26 @@ def test_engines_rebuilding_side_by_side():
     finally:
         for e in engines:
             e.close()
+
+
+def test_a_stalled_rebuild_is_final():
+    """A wait that passes its bound (here no poll at all, so that every kernel
+    leaves at once) ends in an error of its own, and in the same error from
+    then on: no later launch bins on counts that were not cleared, and a list
+    overflow does not take its place."""
+    w = _every_step(W.lj_box(20000, 0.8, 1.0, seed=8))
+    with Engine(w) as e, Engine(w.with_(max_neighbors=1)) as over:
+        for engine in (e, over):
+            engine.initialize(observables=False)
+            assert _members(engine) > 1
+        assert over.stats().overflow == 1
+        for engine in (e, over):
+            _limit(engine, wait_polls=0)
+            engine.advance(24)  # a captured graph and single steps
+            for call in (engine.synchronize, engine.stats, engine.state,
+                         lambda: engine.advance(1), lambda: engine.initialize(False),
+                         engine.neighbors):
+                with pytest.raises(BeadsError, match="lost each other"):
+                    call()
+    # Other engines are untouched.
+    _final_state(_every_step(W.lj_box(5000, 0.8, 1.0, seed=9)), 8)
