@@ -406,8 +406,11 @@ __device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, b
                                    pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
     }
   } else if (lane == 0) {
+    // Entry k as the scatter left it is another workgroup's store (agent_load);
+    // those below k are this lane's own by then.
+    a[b] = agent_load(a + b);
     for (uint32_t k = b + 1; k < e; ++k) {
-      const uint32_t v = a[k];
+      const uint32_t v = agent_load(a + k);
       const real_t xv = p.pos[v].x;
       uint32_t m = k;
       while (m > b && before_in_cell(xv, v, p.pos[a[m - 1]].x, a[m - 1])) {

@@ -71,10 +71,13 @@ def test_more_cells_than_one_prefix():
     _final_state(w, 24)
 
 
-def test_cells_of_more_than_a_wave():
-    w = _every_step(W.lj_box(6000, 0.8, 1.0, seed=4, cutoff=5.0)).with_(max_neighbors=768)
+@pytest.mark.parametrize("n,steps", [(6000, 10), (30000, 48)])
+def test_cells_of_more_than_a_wave(n, steps):
+    """One lane sorts such a cell, from entries that other workgroups scattered
+    (at 30,000 beads over a hundred of them)."""
+    w = _every_step(W.lj_box(n, 0.8, 1.0, seed=4, cutoff=5.0)).with_(max_neighbors=768)
     assert w.n / O.plan(w).n_cells > 64
-    _final_state(w, 10)
+    _final_state(w, steps)
 
 
 def test_engines_rebuilding_side_by_side():
