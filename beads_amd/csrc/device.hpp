@@ -80,6 +80,7 @@ struct alignas(256) Ctrl {
   uint32_t rebuild;         // a rebuild is due in this step
   uint32_t reorder;         // the rebuild also sorts particles into cell order
   uint32_t joined;          // workgroups that joined this step's rebuild (rebuild_kernel)
+  uint32_t outside;         // this rebuild binned an atom outside its cell (outside_cells)
   uint32_t checked;         // a scheduled check ran since the last build
   uint32_t overflow;        // a neighbour list overflowed
   uint32_t stalled;         // a wait inside a rebuild passed its bound: no rebuild or

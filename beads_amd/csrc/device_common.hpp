@@ -179,6 +179,22 @@ __device__ __forceinline__ uint32_t cell_of_position(real4 x, const BoxView& box
   return ix + g.nx * (iy + g.ny * iz);
 }
 
+// Whether the clamp puts x into a cell that does not hold it, on some axis: the
+// wrap leaves a coordinate outside the box by its rounding, which after a
+// displacement of millions of box lengths is a good part of a cell. Up to
+// kOutsideSlack of a cell counts as inside (a build's pruning allows for twice
+// that, kGapSlack); NaN is outside.
+constexpr real_t kOutsideSlack = static_cast<real_t>(1.0 / 128.0);
+__device__ __forceinline__ bool outside_cells(real4 x, const BoxView& box, const CellGridView& g) {
+  auto inside = [](real_t v, real_t lo, real_t inv, uint32_t count) {
+    const real_t s = (v - lo) * inv;
+    return s >= -kOutsideSlack && s <= static_cast<real_t>(count) + kOutsideSlack;
+  };
+  return !(inside(x.x, box.lo[0], g.inv_cell[0], g.nx) &&
+           inside(x.y, box.lo[1], g.inv_cell[1], g.ny) &&
+           inside(x.z, box.lo[2], g.inv_cell[2], g.nz));
+}
+
 // regular_cell_neighbor_builder.cu:40-53.
 __device__ __forceinline__ uint32_t wrapped_axis(uint32_t c, int d, uint32_t count) {
   if (d < 0) return c == 0 ? count - 1 : c - 1;
@@ -287,7 +303,7 @@ constexpr int kRunCodeShift = 28;
 constexpr uint32_t kRunIndexMask = (1u << kRunCodeShift) - 1u;
 
 // The runs of row r (z neighbour r / 3, y neighbour r % 3) of an atom at xi in
-// cell (cx, cy, cz); empty runs are {0, 0}. PRUNE, with 5 or more cells per
+// cell (cx, cy, cz); empty runs are {0, 0}. prune, with 5 or more cells per
 // axis: a row whose cells lie at least gy along y and gz along z from the atom holds
 // neighbours only within ext = sqrt(r_s^2 - gy^2 - gz^2) along x, and none when
 // gy^2 + gz^2 > r_s^2: such rows are dropped, and with x-bin tables (xbins,
@@ -296,15 +312,17 @@ constexpr uint32_t kRunIndexMask = (1u << kRunCodeShift) - 1u;
 // cell). The gaps are taken kGapSlack of a cell short, far above the rounding
 // of the cell coordinates, so a skipped member is farther than ext along x, or
 // than the gaps along y and z, by a margin that no rounding of r^2 closes: the
-// accepted candidates and their order are those of the full scan (of atoms
-// inside the box, as the wrap leaves them; without PRUNE of any).
+// accepted candidates and their order are those of the full scan, provided that
+// the cells hold their members. A member clamped into a face's cell from beyond
+// the face is closer to the cells across it than its bin says, so a caller
+// prunes only where no atom is outside (outside_cells).
 struct RunPair {
   uint2 a, b;
 };
-template <bool PRUNE>
 __device__ inline RunPair row_run_pair(const CellGridView& g, const BoxView& box, real_t rs2,
-                                       const uint32_t* cell_start, const uint4* xbins, real4 xi,
-                                       uint32_t cx, uint32_t cy, uint32_t cz, uint32_t r) {
+                                       const uint32_t* cell_start, const uint4* xbins, bool prune,
+                                       real4 xi, uint32_t cx, uint32_t cy, uint32_t cz,
+                                       uint32_t r) {
   RunPair out;
   out.a = out.b = make_uint2(0u, 0u);
   const int iz = static_cast<int>(r / 3), iy = static_cast<int>(r % 3);
@@ -339,8 +357,9 @@ __device__ inline RunPair row_run_pair(const CellGridView& g, const BoxView& box
   uint32_t skip = 0, keep = 0xffffffffu;  // members dropped at the row's start, kept of its last cell
   uint32_t n_last = 0;
   const uint32_t last = rowc + (m1 >= m0 ? m1 : l1);
-  if (PRUNE && g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
+  if (prune && g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
     constexpr real_t kGapSlack = static_cast<real_t>(1.0 / 64.0);
+    static_assert(kGapSlack >= 2 * kOutsideSlack, "a member counted inside stays within the slack");
     const real_t fy = (xi.y - box.lo[1]) * g.inv_cell[1] - static_cast<real_t>(cy);
     const real_t fz = (xi.z - box.lo[2]) * g.inv_cell[2] - static_cast<real_t>(cz);
     // Gap to the row below (k = 0) and above (k = 2) along one axis.
@@ -386,10 +405,11 @@ __device__ inline RunPair row_run_pair(const CellGridView& g, const BoxView& box
 // A team's runs in visiting order, empty ones left out, into its LDS entry
 // list (kMaxRuns entries); returns how many, the same in every lane. Lane t of
 // TEAM evaluates rows t, t + TEAM, ... Every lane of the team calls it.
-template <int TEAM, bool PRUNE>
+template <int TEAM>
 __device__ inline uint32_t team_runs(const CellGridView& g, const BoxView& box, real_t rs2,
-                                     const uint32_t* cell_start, const uint4* xbins, real4 xi,
-                                     uint32_t c, uint32_t t, uint32_t team_lane0, uint2* runs) {
+                                     const uint32_t* cell_start, const uint4* xbins, bool prune,
+                                     real4 xi, uint32_t c, uint32_t t, uint32_t team_lane0,
+                                     uint2* runs) {
   const uint32_t cx = c % g.nx, cyz = c / g.nx, cy = cyz % g.ny, cz = cyz / g.ny;
   constexpr uint64_t kTeamMask = TEAM >= 64 ? ~0ull : (1ull << TEAM) - 1ull;
   uint32_t n = 0;
@@ -398,7 +418,7 @@ __device__ inline uint32_t team_runs(const CellGridView& g, const BoxView& box, 
     RunPair p;
     p.a = p.b = make_uint2(0u, 0u);
     if (r0 + t < static_cast<uint32_t>(kRows)) {
-      p = row_run_pair<PRUNE>(g, box, rs2, cell_start, xbins, xi, cx, cy, cz, r0 + t);
+      p = row_run_pair(g, box, rs2, cell_start, xbins, prune, xi, cx, cy, cz, r0 + t);
     }
     const bool has_a = p.a.y != 0, has_b = p.b.y != 0;  // a nonempty run ends past 0
     const uint64_t ma = (__ballot(has_a) >> team_lane0) & kTeamMask;

@@ -1193,8 +1193,9 @@ void Engine::frame_load(const real_t* positions_dev, bool reuse_list, bool async
   frame_loaded_ = false;
   load_frame(positions_dev, reuse_list);
   // The force pass normally clears the rebuild flags; no force pass runs here.
-  static_assert(offsetof(Ctrl, joined) == 2 * sizeof(uint32_t), "rebuild, reorder, joined lead Ctrl");
-  BEADS_HIP(hipMemsetAsync(ctrl_.data(), 0, 3 * sizeof(uint32_t), stream_));
+  static_assert(offsetof(Ctrl, outside) == 3 * sizeof(uint32_t),
+                "rebuild, reorder, joined, outside lead Ctrl");
+  BEADS_HIP(hipMemsetAsync(ctrl_.data(), 0, 4 * sizeof(uint32_t), stream_));
   BEADS_HIP(hipGetLastError());
   if (!async) check_overflow(fetch_ctrl());
   frame_loaded_ = true;

@@ -272,10 +272,12 @@ __device__ __forceinline__ uint32_t block_exclusive(uint32_t v, uint32_t* lds, u
 
 // cell_list_build.cu:135-166: cell index in the storage precision and atomic
 // counts, one atomic per distinct cell of the wave.
-__device__ __forceinline__ void bin_atom(const CellScanParams& p, uint32_t i) {
-  const uint32_t c = cell_of_position(p.pos[i], p.box, p.grid);
+__device__ __forceinline__ void bin_atom(const CellScanParams& p, Ctrl* ctrl, uint32_t i) {
+  const real4 x = p.pos[i];
+  const uint32_t c = cell_of_position(x, p.box, p.grid);
   p.cell_of[i] = c;
   wave_increment(p.cell_count, c);
+  raise_flag(outside_cells(x, p.box, p.grid), &ctrl->outside);
 }
 
 // Cells up to which a member sums the counts before its own tile by itself
@@ -630,7 +632,7 @@ __global__ __launch_bounds__(kRebuildBlock) void rebuild_kernel(CellScanParams c
   const uint32_t n = cp.n;
   const uint32_t first = m.rank * kRebuildBlock + threadIdx.x;
   const uint32_t stride = m.count * kRebuildBlock;
-  for (uint64_t i = first; i < n; i += stride) bin_atom(cp, static_cast<uint32_t>(i));
+  for (uint64_t i = first; i < n; i += stride) bin_atom(cp, ctrl, static_cast<uint32_t>(i));
   if (!member_barrier<false>(ctrl, m)) return;
   // Every member has read the counters that its decisions come from.
   if (m.rank == 0) {
@@ -659,15 +661,15 @@ constexpr uint32_t kBuildAtoms = kBlock / kBuildTeam;
 // runs (more LDS per workgroup costs occupancy).
 constexpr uint32_t kStageBytesMax = 24576;
 
-// Rows path: regular grid, at least 5 cells per axis, atom i not in an
-// x-boundary cell, so that each row is one run. Writes row r's run for r = t,
+// Rows path: regular grid, at least 5 cells per axis, no atom outside the
+// cells, atom i not in an x-boundary cell, so that each row is one run. Writes row r's run for r = t,
 // t + kBuildTeam, ... (the team's lanes share the rows), widens the block's
 // span of row r, [lo[r], hi[r]), to cover a nonempty run, and returns false
 // off the rows path.
 __device__ inline bool row_runs(const BuildParams& p, uint32_t i, uint32_t t, uint2* rows,
                                 uint32_t* lo_r, uint32_t* hi_r) {
   const CellGridView& g = p.grid;
-  if (g.path != 1 || g.nx < 5 || g.ny < 5 || g.nz < 5) return false;
+  if (g.path != 1 || g.nx < 5 || g.ny < 5 || g.nz < 5 || p.ctrl->outside != 0) return false;
   const uint32_t c = p.cell_of[i];
   const uint32_t cx = c % g.nx, cyz = c / g.nx, cy = cyz % g.ny, cz = cyz / g.ny;
   if (cx < 1 || cx + 1 >= g.nx) return false;
@@ -675,7 +677,7 @@ __device__ inline bool row_runs(const BuildParams& p, uint32_t i, uint32_t t, ui
 #pragma unroll 1
   for (uint32_t r = t; r < static_cast<uint32_t>(kRows); r += kBuildTeam) {
     const uint2 d =
-        row_run_pair<true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r).a;
+        row_run_pair(g, p.box, p.rs2, p.cell_start, p.cell_xbins, true, xi, cx, cy, cz, r).a;
     rows[r] = d;
     const uint32_t b = d.x, e = d.y & kRunIndexMask;
     if (b < e) {
@@ -949,13 +951,16 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
           k += kBuildTeam * kBuildSlots;
         }
       };
-      // Boundary cells and grids of fewer than 5 cells per axis: the rows one
-      // after another, each one run or two.
+      // Boundary cells, grids of fewer than 5 cells per axis, and any grid while
+      // some atom is outside the cells (then nothing is pruned, and a wrapped
+      // cell says nothing about the image): the rows one after another, each
+      // one run or two.
+      const bool pruned = p.ctrl->outside == 0;
       auto rows_in_turn = [&](auto mode) {
 #pragma unroll 1
         for (uint32_t r = 0; r < static_cast<uint32_t>(kRows); ++r) {
-          const RunPair q =
-              row_run_pair<true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi, cx, cy, cz, r);
+          const RunPair q = row_run_pair(g, p.box, p.rs2, p.cell_start, p.cell_xbins, pruned, xi,
+                                         cx, cy, cz, r);
 #pragma unroll 1
           for (int part = 0; part < 2; ++part) {
             const uint2 d = part == 0 ? q.a : q.b;
@@ -970,7 +975,7 @@ __global__ __launch_bounds__(kBlock) void build_kernel(BuildParams p) {
         scan_rows([](uint32_t k0, int u) { return stage[k0 + u * kBuildTeam]; });
       } else if (rows_path) {
         scan_rows(entry);
-      } else if (g.path == 1 && g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
+      } else if (pruned && g.path == 1 && g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
         rows_in_turn(kShiftMode{});
       } else {
         rows_in_turn(kGenericMode{});
@@ -1009,6 +1014,7 @@ __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
   const uint32_t q = xcd_block(blockIdx.x, gridDim.x) * kWideAtoms + threadIdx.x / TEAM;
   uint2* const runs = run_lds + (threadIdx.x / TEAM) * kMaxRuns;
   const bool direct = p.grid.path == 0;
+  const bool pruned = p.ctrl->outside == 0;  // as in build_kernel
   const CellGridView& g = p.grid;
   real4 xi = make_real4(0, 0, 0, 0);
   uint32_t i = q, n_runs = 0, count = 0;
@@ -1020,8 +1026,8 @@ __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
     } else {
       xi = p.cell_pos[q];  // the atom's position, .w its slot
       i = id_of(xi.w);
-      n_runs = team_runs<TEAM, true>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, xi,
-                                    cell_of_position(xi, p.box, g), t, team_lane0, runs);
+      n_runs = team_runs<TEAM>(g, p.box, p.rs2, p.cell_start, p.cell_xbins, pruned, xi,
+                               cell_of_position(xi, p.box, g), t, team_lane0, runs);
     }
   }
   __syncthreads();
@@ -1049,7 +1055,7 @@ __global__ __launch_bounds__(kBlock) void build_wide_kernel(BuildParams p) {
         return *reinterpret_cast<const real4*>(cp_bytes +
                                                k * static_cast<uint32_t>(sizeof(real4)));
       };
-      if (g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
+      if (pruned && g.nx >= 5 && g.ny >= 5 && g.nz >= 5) {
         count = scan_runs<TEAM, kWideSlots>(runs, n_runs, t, team_lane0, p.box, entry, accept,
                                                  put, kShiftMode{});
       } else {
@@ -1399,6 +1405,7 @@ __global__ __launch_bounds__(kBlock) void force_kernel(ForceParams p) {
     p.ctrl->rebuild = 0;
     p.ctrl->reorder = 0;
     p.ctrl->joined = 0;
+    p.ctrl->outside = 0;
   }
   const LjCoeff c0 = TYPES == 0 && !HALF ? p.lj[0] : LjCoeff{0.0, 0.0, 0.0, 0.0};
   const uint32_t t = threadIdx.x & (TEAM - 1);

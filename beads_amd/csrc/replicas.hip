@@ -842,8 +842,9 @@ __global__ __launch_bounds__(kPhasedBlock) void phased_build_kernel(ReplicaParam
         if (t == 0) runs[0] = make_uint2(0u, n);
         n_runs = 1;
       } else {
-        n_runs = team_runs<kPhasedBuildTeam, false>(g, d.box, d.rs2, A.cell_start + d.cell0, nullptr, xi,
-                                             A.cell_of[d.atom0 + i], t, team_lane0, runs);
+        n_runs = team_runs<kPhasedBuildTeam>(g, d.box, d.rs2, A.cell_start + d.cell0, nullptr,
+                                             false, xi, A.cell_of[d.atom0 + i], t, team_lane0,
+                                             runs);
       }
     }
     __syncthreads();
