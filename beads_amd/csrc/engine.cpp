@@ -1193,9 +1193,11 @@ void Engine::frame_load(const real_t* positions_dev, bool reuse_list, bool async
   frame_loaded_ = false;
   load_frame(positions_dev, reuse_list);
   // The force pass normally clears the rebuild flags; no force pass runs here.
+  // A kernel and not a memset: no memset node goes into a graph that a caller
+  // captures, and with `joined` left over nobody would join the next rebuild.
   static_assert(offsetof(Ctrl, outside) == 3 * sizeof(uint32_t),
                 "rebuild, reorder, joined, outside lead Ctrl");
-  BEADS_HIP(hipMemsetAsync(ctrl_.data(), 0, 4 * sizeof(uint32_t), stream_));
+  launch_fill_f64(reinterpret_cast<double*>(ctrl_.data()), 2, stream_);
   BEADS_HIP(hipGetLastError());
   if (!async) check_overflow(fetch_ctrl());
   frame_loaded_ = true;
