@@ -273,7 +273,8 @@ beads_status_t beads_engine_frame_backward_noalloc(beads_engine_t* e, const bead
 }
 
 // Not part of the API (undeclared in beads_amd.h): what tests need to force a
-// rebuild that only some workgroups share, or one that stalls.
+// rebuild that only some workgroups share, or one that stalls, and a state read
+// in small windows.
 beads_status_t beads_internal_rebuild_limits(beads_engine_t* e, uint32_t members,
                                              int64_t join_ticks, uint32_t wait_polls) {
   return guarded([&] {
@@ -290,6 +291,11 @@ beads_status_t beads_internal_rebuild_members(beads_engine_t* e, uint32_t* membe
     beads_amd::require(members != nullptr, "members output is null");
     *members = engine_of(e).rebuild_members();
   });
+}
+
+beads_status_t beads_internal_state_sizes(beads_engine_t* e, uint64_t whole, uint64_t window,
+                                          uint64_t piece) {
+  return guarded([&] { engine_of(e).state_reader().set_sizes(whole, window, piece); });
 }
 
 void beads_engine_destroy(beads_engine_t* e) {

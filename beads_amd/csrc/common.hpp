@@ -139,6 +139,7 @@ class PinnedBuffer {
       if (ptr_ != nullptr) {
         (void)hipHostFree(ptr_);
         ptr_ = nullptr;
+        cap_ = 0;
       }
       void* p = nullptr;
       BEADS_HIP(hipHostMalloc(&p, count * sizeof(T), hipHostMallocDefault));

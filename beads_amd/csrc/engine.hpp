@@ -132,6 +132,7 @@ class Engine {
   // stalled one, and how many shared the last rebuild.
   void set_rebuild_limits(const RebuildLimits& limits);
   uint32_t rebuild_members();
+  StateReader& state_reader() { return state_reader_; }
   uint32_t n_particles() const { return n_; }
   int32_t n_types() const { return n_types_; }
   int32_t n_bond_types() const { return n_bond_types_; }

@@ -492,6 +492,7 @@ __global__ __launch_bounds__(kBlock) void pack_state_kernel(PackStateParams p) {
   if (i >= p.n) {
     return;
   }
+  const uint32_t a = p.first + i;
   auto put3 = [&](uint64_t field, auto x, auto y, auto z) {
     auto* o = reinterpret_cast<decltype(x)*>(p.out + field) + 3 * static_cast<size_t>(i);
     o[0] = x;
@@ -499,28 +500,28 @@ __global__ __launch_bounds__(kBlock) void pack_state_kernel(PackStateParams p) {
     o[2] = z;
   };
   if (p.positions != kNoField || p.types != kNoField) {
-    const real4 x = p.pos[i];
+    const real4 x = p.pos[a];
     if (p.positions != kNoField) put3(p.positions, x.x, x.y, x.z);
     if (p.types != kNoField) {
       reinterpret_cast<int32_t*>(p.out + p.types)[i] = static_cast<int32_t>(id_of(x.w)) + 1;
     }
   }
   if (p.velocities != kNoField || p.masses != kNoField) {
-    const real4 v = p.vel[i];
+    const real4 v = p.vel[a];
     if (p.velocities != kNoField) put3(p.velocities, v.x, v.y, v.z);
     if (p.masses != kNoField) reinterpret_cast<real_t*>(p.out + p.masses)[i] = v.w;
   }
   if (p.forces != kNoField) {
-    const real4 f = p.force[i];
+    const real4 f = p.force[a];
     put3(p.forces, f.x, f.y, f.z);
   }
   if (p.images != kNoField) {
-    const int4 m = p.image[i];
+    const int4 m = p.image[a];
     put3(p.images, m.x, m.y, m.z);
   }
-  if (p.tags != kNoField) reinterpret_cast<uint32_t*>(p.out + p.tags)[i] = p.tag[i];
+  if (p.tags != kNoField) reinterpret_cast<uint32_t*>(p.out + p.tags)[i] = p.tag[a];
   if (p.molecule_ids != kNoField) {
-    reinterpret_cast<uint32_t*>(p.out + p.molecule_ids)[i] = p.molid[i];
+    reinterpret_cast<uint32_t*>(p.out + p.molecule_ids)[i] = p.molid[a];
   }
 }
 

@@ -100,11 +100,11 @@ struct PackParams {
 };
 void launch_pack_records(const PackParams& p, hipStream_t stream);
 
-// The state as arrays of one field each: byte offsets into out (kNoField: not
-// wanted).
+// The state of n atoms from `first` on as arrays of one field each: byte
+// offsets into out (kNoField: not wanted).
 constexpr uint64_t kNoField = ~uint64_t{0};
 struct PackStateParams {
-  uint32_t n;
+  uint32_t first, n;
   const real4* pos;
   const real4* vel;
   const real4* force;

@@ -1,4 +1,4 @@
-// Device state to host arrays: one packing kernel, staged copies, and for large
+// Device state to host arrays: a packing kernel, staged copies, and for large
 // states several host threads, each filling its part of the caller's arrays
 // while the next parts are on their way.
 #pragma once
@@ -14,6 +14,8 @@
 
 namespace beads_amd {
 
+struct PackStateParams;
+
 // The per-atom device arrays of one system (null tag / molid: not available).
 struct StateSource {
   uint32_t n = 0;
@@ -27,7 +29,7 @@ struct StateSource {
 
 class StateReader {
  public:
-  StateReader() = default;
+  StateReader();
   ~StateReader();
   StateReader(const StateReader&) = delete;
   StateReader& operator=(const StateReader&) = delete;
@@ -36,15 +38,30 @@ class StateReader {
   // on return.
   void read(const StateSource& src, const beads_state_out_t& out, hipStream_t stream);
 
- private:
-  struct Field {  // bytes [offset, offset + size) of the staged state go to dst
-    size_t offset, size;
-    unsigned char* dst;
-  };
-  static void deliver(const std::vector<Field>& fields, const unsigned char* bytes, size_t offset,
-                      size_t size);
-  void deliver_in_chunks(const std::vector<Field>& fields, size_t total, hipStream_t stream);
+  // The most a read copies at once, the most it stages on the device, and the
+  // size of a copy above the first.
+  void set_sizes(size_t whole, size_t window, size_t piece);
 
+ private:
+  // A wanted field: its bytes per atom, the caller's array, and where the
+  // packing kernel is told the field's place in a window.
+  struct Field {
+    size_t bytes;
+    unsigned char* dst;
+    uint64_t PackStateParams::* place;
+  };
+  // The atoms staged on the device together (the last window may hold fewer).
+  struct Window {
+    size_t first, count;
+  };
+  size_t reserve(size_t n, size_t per_atom);
+  void pack(const std::vector<Field>& fields, PackStateParams p, Window w, hipStream_t stream);
+  static void deliver(const std::vector<Field>& fields, Window w, const unsigned char* bytes,
+                      size_t offset, size_t size);
+  void read_windows(const std::vector<Field>& fields, const PackStateParams& p, size_t per_atom,
+                    size_t window_atoms, hipStream_t stream);
+
+  size_t whole_bytes_, window_bytes_, piece_bytes_;
   DeviceBuffer<unsigned char> stage_;
   PinnedBuffer<unsigned char> host_;
   std::vector<hipEvent_t> events_;

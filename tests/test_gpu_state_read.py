@@ -1,4 +1,4 @@
-"""Reading the state back: the single copy, the copy in chunks by several
+"""Reading the state back: the single copy, the copy in pieces by several
 threads, and subsets of the fields give back exactly what the run was created
 with (before its first step nothing has touched it)."""
 
@@ -27,9 +27,11 @@ def _inputs(n: int) -> W.Workload:
 
 
 # 64 bytes an atom in binary32, 104 in binary64: 65,536 and 40,329 atoms are the
-# last in one copy; chunks of 1 MB are whole at 81,920 atoms.
+# last in one copy; pieces of 1 MB are whole at 81,920, windows of 16 MB at
+# 524,288.
 @pytest.mark.parametrize("precision,n", [("single", 500), ("single", 65536), ("single", 65537),
                                          ("single", 81920), ("single", 131071),
+                                         ("single", 524288), ("single", 524289),
                                          ("double", 40329), ("double", 40330)])
 def test_state_is_what_went_in(precision, n):
     w = _inputs(n)
@@ -41,6 +43,25 @@ def test_state_is_what_went_in(precision, n):
             for k in FIELDS:
                 assert np.array_equal(s[k], getattr(w, k)), k
             assert not s["forces"].any()
+
+
+# Windows as small as they get where the card is full: a few and many, pieces
+# that divide a window and pieces that do not, one piece a window.
+@pytest.mark.parametrize("precision,n,window,piece", [
+    ("single", 500, 1 << 14, 1 << 14), ("single", 700, 1 << 14, 1000),
+    ("single", 20001, 1 << 14, 1 << 12), ("single", 20001, 100000, 1 << 20),
+    ("double", 20001, 20000, 4096)])
+def test_small_windows(precision, n, window, piece):
+    w = _inputs(n)
+    if precision == "double":
+        w = w.as_float64(jitter=1e-9)
+    with capi.Engine(w, precision) as e:
+        e._check(e.lib.beads_internal_state_sizes(e.handle, C.c_uint64(0), C.c_uint64(window),
+                                                  C.c_uint64(piece)))
+        for _ in range(2):
+            s = e.state()
+            for k in FIELDS:
+                assert np.array_equal(s[k], getattr(w, k)), k
 
 
 @pytest.mark.parametrize("n", [500, 131071])
