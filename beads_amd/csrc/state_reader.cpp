@@ -4,7 +4,6 @@
 #include <cstdint>
 #include <cstring>
 #include <exception>
-#include <mutex>
 #include <system_error>
 #include <thread>
 
@@ -41,6 +40,7 @@ StateReader::~StateReader() {
 void StateReader::set_sizes(size_t whole, size_t window, size_t piece) {
   require(window >= kSmallest && piece > 0, "state windows hold at least " +
                                                 std::to_string(kSmallest) + " bytes.");
+  const std::lock_guard<std::mutex> lock(mutex_);
   whole_bytes_ = whole;
   window_bytes_ = window;
   piece_bytes_ = piece;
@@ -169,6 +169,7 @@ void StateReader::read_windows(const std::vector<Field>& fields, const PackState
 }
 
 void StateReader::read(const StateSource& src, const beads_state_out_t& o, hipStream_t stream) {
+  const std::lock_guard<std::mutex> lock(mutex_);
   std::vector<Field> fields;
   size_t per_atom = 0;
   PackStateParams p{};

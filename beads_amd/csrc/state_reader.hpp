@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstddef>
+#include <mutex>
 #include <vector>
 
 #include "beads_amd.h"
@@ -35,7 +36,7 @@ class StateReader {
   StateReader& operator=(const StateReader&) = delete;
 
   // Fills the non-null arrays of out in the stream's order; they are complete
-  // on return.
+  // on return. Callable from several threads, one read at a time.
   void read(const StateSource& src, const beads_state_out_t& out, hipStream_t stream);
 
   // The most a read copies at once, the most it stages on the device, and the
@@ -61,6 +62,7 @@ class StateReader {
   void read_windows(const std::vector<Field>& fields, const PackStateParams& p, size_t per_atom,
                     size_t window_atoms, hipStream_t stream);
 
+  std::mutex mutex_;
   size_t whole_bytes_, window_bytes_, piece_bytes_;
   DeviceBuffer<unsigned char> stage_;
   PinnedBuffer<unsigned char> host_;

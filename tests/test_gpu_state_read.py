@@ -1,10 +1,12 @@
 """Reading the state back: the single copy, the copy in pieces by several
-threads, and subsets of the fields give back exactly what the run was created
-with (before its first step nothing has touched it)."""
+threads, subsets of the fields and reads from several threads at once give back
+exactly what the run was created with (before its first step nothing has touched
+it)."""
 
 from __future__ import annotations
 
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -62,6 +64,27 @@ def test_small_windows(precision, n, window, piece):
             s = e.state()
             for k in FIELDS:
                 assert np.array_equal(s[k], getattr(w, k)), k
+
+
+@pytest.mark.parametrize("n", [500, 200000])
+def test_reads_from_several_threads(n):
+    w = _inputs(n)
+    wrong = []
+    with capi.Engine(w, "single") as e:
+        def read(k):
+            try:
+                for _ in range(6):
+                    s = e.state()
+                    if not all(np.array_equal(s[f], getattr(w, f)) for f in FIELDS):
+                        wrong.append(k)
+            except Exception as x:  # noqa: BLE001
+                wrong.append(x)
+        threads = [threading.Thread(target=read, args=(k,)) for k in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert not wrong
 
 
 @pytest.mark.parametrize("n", [500, 131071])
