@@ -1,7 +1,7 @@
 """The rebuild kernel's phases (binning, scan, scatter, sort, reorder in one
 launch) where its work splits differently: part-filled and single workgroups,
 more cells than a workgroup sums the prefix of by itself, cells of more than a
-wave's members.
+wave's members, workgroups that came too late to take part.
 
 Every step rebuilds and reorders (zero skin, sort at every build), so each phase
 hands over to the next many times before the final cells, in-cell order and
@@ -80,10 +80,41 @@ def test_cells_of_more_than_a_wave(n, steps):
     _final_state(w, steps)
 
 
+@pytest.mark.parametrize("members,join_ticks", [(1, 3000), (2, 3000), (37, 3000), (256, 0)])
+def test_rebuilds_that_part_of_the_grid_shares(members, join_ticks):
+    """The list of a rebuild's workgroups closed before all are on it, as beside
+    another stream's kernels (at a count, so that the split is known, and at
+    once): those on it do the whole of every phase, reorders with listed terms
+    among them, and the others leave."""
+    w = _every_step(W.polymer_melt(n_chains=300, beads_per_chain=50, seed=7))
+    assert O.plan(w).path != 0
+    got = []
+    for limits in ({}, dict(members=members, join_ticks=join_ticks)):
+        with Engine(w) as e:
+            e.initialize(observables=False)
+            full = _members(e)
+            _limit(e, **limits)
+            e.advance(20, observables_on_last=True)  # a captured graph and single steps
+            took = _members(e)
+            st, cells, stats = e.state(), e.cells(O.plan(w).n_cells), e.stats()
+            counts, lst = e.neighbors()
+        assert stats.overflow == 0 and stats.build_count == 21 and stats.reorder_count >= 20
+        assert full > 37
+        if limits and join_ticks:  # closed at once: as many as had started
+            assert took == members
+        got.append((st, cells, counts, list(stats.pe),
+                    np.where(np.arange(len(lst))[:, None] < counts[None], lst, 0)))
+    (sa, ca, na, pa, la), (sb, cb, nb, pb, lb) = got
+    for k in sa:
+        assert np.array_equal(sa[k], sb[k]), k
+    for k in ca:
+        assert np.array_equal(ca[k], cb[k]), k
+    assert np.array_equal(na, nb) and np.array_equal(la, lb) and pa == pb
+
+
 def test_engines_rebuilding_side_by_side():
     """Several engines step on their own streams at once, each rebuilding every
-    step: whichever workgroups of a rebuild the GPU holds, the result is that of
-    the engine alone."""
+    step: the result is that of the engine alone."""
     ws = [_every_step(W.lj_box(n, 0.8, 1.0, seed=n)) for n in (3000, 40000, 20000, 60000)]
     alone = []
     for w in ws:
