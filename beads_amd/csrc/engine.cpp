@@ -736,6 +736,7 @@ void Engine::set_up_params() {
   rb.neighbor_parts = neighbor_parts_.data();
   rb.sync_lines = sync_lines_.data();
   rb.tile_sums = tile_sums_.data();
+  rb.limits.join_ticks = rebuild_join_ticks(n_);
   rb.stalled_host = stalled_host_.data();
 
   ReorderParams& r = reorder_params_;

@@ -32,12 +32,26 @@ constexpr uint32_t kSyncLine = 16;  // 8-byte words of a member's arrival or rel
 struct RebuildLimits {
   uint32_t members = kRebuildMaxBlocks;  // most that take part
   int64_t join_ticks = 3000;             // how long the first waits for the grid to start,
-                                         // in wall_clock64 ticks (100 MHz)
+                                         // in wall_clock64 ticks (rebuild_join_ticks)
   // Polls before any other wait is given up: at about a microsecond each over
   // 4 s of running. Polls and not time, which passes for a workgroup whose
   // queue is off the GPU too.
   uint32_t wait_polls = 1u << 22;
 };
+
+// Ticks of 10 ns. An idle GPU starts the grid in a few microseconds; beside
+// another stream's kernels a rebuild of a large system by half the grid costs
+// more than the wait. Next to copies that fill the GPU (x *= 1 over 1 GiB), 96
+// steps of an LJ fluid with 17 rebuilds and 2 reorders, ms by window of 0 / 10 /
+// 30 / 100 / 200 us: 4,000,000 beads 234 / 190 / 170 / 163.6 / 162.9 (half the
+// grid joins in 30 us, all of it in 200), 1,000,000 beads 59.7 / 57.4 / 54.2 /
+// 52.8 to 54.1 / 55.1. As seven launches, which start as the GPU comes free,
+// these were 162.0 and 49.5 (engine and copies together 225 and 57.6 against
+// 222 and 56.7). At 48,000 beads 30 us is as long as a rebuild takes (12.1 ms,
+// 14.6 as seven launches).
+constexpr int64_t rebuild_join_ticks(uint32_t n) {
+  return n < 300000 ? 3000 : (n < 2000000 ? n / 100 : 20000);
+}
 
 struct RebuildParams {
   Ctrl* ctrl;
