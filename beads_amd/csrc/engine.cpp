@@ -1221,6 +1221,7 @@ void Engine::frame_backward(const real_t* grad_forces_dev, double grad_energy,
   if (models_.dihedral) models_.dihedral->bind_adjoint(p);
   const size_t n_params = adjoint_param_count();
   real4* staging = nullptr;
+  bool interleaved = !noalloc;  // the static scratch holds dL/dF alone
   if (noalloc) {
     require(n_ <= kNoAllocMaxAtoms,
             "frame_backward_noalloc serves at most " + std::to_string(kNoAllocMaxAtoms) +
@@ -1229,7 +1230,17 @@ void Engine::frame_backward(const real_t* grad_forces_dev, double grad_energy,
     staging = scratch_address();
     async = true;
   } else {
-    grad_force4_.resize(2 * static_cast<size_t>(n_));  // interleaved with the positions
+    // Interleaved with the positions where the card has room for both.
+    const size_t n = n_;
+    if (grad_force4_.size() == 0) {
+      try {
+        grad_force4_.resize(2 * n);
+      } catch (const Error&) {
+        (void)hipGetLastError();
+        grad_force4_.resize(n);
+      }
+    }
+    interleaved = grad_force4_.size() == 2 * n;
     staging = grad_force4_.data();
   }
   if (noalloc) {
@@ -1240,14 +1251,14 @@ void Engine::frame_backward(const real_t* grad_forces_dev, double grad_energy,
     BEADS_HIP(hipMemsetAsync(grad_params_dev, 0, n_params * sizeof(double), stream_));
   }
   p.n = n_;
-  if (noalloc) {  // its static scratch holds dL/dF alone
-    launch_pack_xyz(n_, grad_forces_dev, staging, stream_);
-    p.pos = pos_.data();
-    p.g = staging;
-  } else {
+  if (interleaved) {
     launch_pack_frame(n_, pos_.data(), grad_forces_dev, staging, stream_);
     p.pos = staging;
     p.g = staging + 1;
+  } else {
+    launch_pack_xyz(n_, grad_forces_dev, staging, stream_);
+    p.pos = pos_.data();
+    p.g = staging;
   }
   p.nbr_count = nbr_count_.data();
   p.nbr = nbr_.data();
@@ -1267,7 +1278,7 @@ void Engine::frame_backward(const real_t* grad_forces_dev, double grad_energy,
   p.grad_energy = grad_energy;
   p.grad_pos = grad_positions_dev;
   p.grad_params = grad_params_dev;
-  launch_fm_backward(p, !noalloc, stream_);
+  launch_fm_backward(p, interleaved, stream_);
   BEADS_HIP(hipGetLastError());
   if (noalloc) return;
   BEADS_HIP(hipEventRecord(frame_events_[3], stream_));
