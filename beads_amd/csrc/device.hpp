@@ -89,7 +89,7 @@ struct alignas(256) Ctrl {
   uint64_t build_count;
   uint64_t dangerous;
   uint64_t reorder_count;
-  uint64_t clock;           // steps advanced (counted by the control kernel)
+  uint64_t clock;           // steps advanced (update_control)
   uint64_t last_sort;       // clock at the last reorder
   double lambda;            // Berendsen factor still to be applied to vel
   double ke_pre;            // kinetic energy after the post-force half-kick
@@ -158,8 +158,6 @@ struct ForceParams {
   double* partials;       // per block: ke, pe[4], vir[4]
   int32_t sums;           // form them (set by launch_force)
   Ctrl* ctrl;
-  uint32_t* cell_count;   // zeroed after a rebuild consumed it
-  uint32_t n_cells;
   int32_t half;           // stored list holds each pair once (j > i)
   double* pair_acc;       // [3 N] LJ sums of the half-list pair pass
 };
@@ -189,10 +187,8 @@ struct BuildParams {
   real_t rs2;
   const uint32_t* cell_of;
   const uint32_t* cell_start;
-  const uint32_t* cell_count;
-  const uint32_t* cell_atoms;
-  const real4* cell_pos;  // cell_atoms' positions, .w = the slot's bits
-  const uint4* cell_xbins; // per cell: x-bin prefix counts (cell_sort_kernel)
+  const real4* cell_pos;  // positions in cell order, .w = the slot's bits
+  const uint4* cell_xbins; // per cell: x-bin prefix counts (sort_cell)
   const uint32_t* topo_count;
   const uint32_t* excl;
   uint32_t ecap;

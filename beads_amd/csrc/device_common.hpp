@@ -93,7 +93,7 @@ __device__ __forceinline__ double team_sum(double v) {
 // order. Lanes whose key has not come up by then add for themselves: spatially
 // sorted atoms of a wave lie in a handful of cells, but atoms in a caller's
 // order have a cell each, and one returning atomic after another is a chain of
-// up to 64 memory latencies (cell_scatter of 100,000 shuffled beads). Returns
+// up to 64 memory latencies (the scatter of 100,000 shuffled beads). Returns
 // the counter's value before this lane's increment.
 constexpr int kSharedKeys = 6;
 

@@ -662,8 +662,6 @@ void Engine::set_up_params() {
   f.dof = std::max(0.0, 3.0 * static_cast<double>(n_) - 3.0);
   f.partials = partials_.data();
   f.ctrl = ctrl_.data();
-  f.cell_count = cell_count_.data();
-  f.n_cells = plan_.n_cells;
   f.half = half_list_ ? 1 : 0;
   f.pair_acc = pair_acc_.data();
 
@@ -700,8 +698,6 @@ void Engine::set_up_params() {
   b.rs2 = plan_.search_cutoff_sq;
   b.cell_of = cell_of_.data();
   b.cell_start = cell_start_.data();
-  b.cell_count = cell_count_.data();
-  b.cell_atoms = cell_atoms_.data();
   b.cell_pos = cell_pos_.data();
   b.cell_xbins = cell_xbins_.data();
   b.topo_count = topo_count_.data();

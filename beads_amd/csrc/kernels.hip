@@ -341,7 +341,7 @@ __device__ __forceinline__ void scatter_atom(const CellScanParams& p, uint32_t i
 // rank; the x-bin prefix counts come from one ballot per bin. A larger cell
 // is insertion-sorted by lane 0. When no reorder follows, the kernel also
 // writes the members' positions in cell order with the slot in .w (the
-// build's candidate stream); after a reorder, reorder_commit writes them.
+// build's candidate stream); after a reorder, commit_atom writes them.
 __device__ __forceinline__ real4 cell_entry(real4 x, uint32_t slot) {
   return make_real4(x.x, x.y, x.z, real_of_id(slot));
 }
@@ -1565,10 +1565,15 @@ void launch_pack_records(const PackParams& p, hipStream_t stream) {
 
 // Atoms up to which the wide build is used, and its 32-lane shape. Measured,
 // 4 lanes / 16 / 32, us per build (equilibrated systems): LJ fluid of 4,000
-// beads 65 / 18 / 14, of 32,000 64 / 34 / 39; bead-spring melt of 8,000
-// 96 / 24 / 21, of 48,000 106 / 58 / 67, of 100,000 140 / 100 / 122; four-type
-// mixture of 100,000 75 / 65 / 92. Above, 4 / 16 lanes with four slots: melt of
-// 216,000 205 / 204, of 512,000 384 / 440; mixture of 216,000 119 / 139.
+// beads 65 / 18 / 14, of 32,000 65 / 32 / 39; bead-spring melt of 8,000
+// 96 / 24 / 21, of 48,000 103 / 58 / 67. 4 / 16 around the upper line: melt of
+// 100,000 144 / 100, of 150,000 166 / 140, of 216,000 210 / 196, of 288,000
+// 247 / 255; fluid of 108,000 99 / 82, of 144,000 112 / 106, of 256,000
+// 162 / 175; mixture of 100,000 77 / 66, of 150,000 96 / 91, of 216,000
+// 124 / 125, of 288,000 150 / 162; solvent in a caller's order of 100,000
+// 138 / 101, of 150,000 168 / 143, of 216,000 214 / 206, of 288,000 257 / 264.
+// The upper line was set when nothing larger than 100,000 had been timed with
+// two slots a round; by these figures it belongs at about 200,000.
 constexpr uint32_t kWideBuild32Max = 12000;
 constexpr uint32_t kWideBuildMax = 100000;
 
