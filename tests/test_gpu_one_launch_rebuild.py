@@ -44,7 +44,7 @@ def _final_state(w, steps):
         assert np.array_equal(np.sort(lst[:counts[i], i]), np.sort(rl[i, :rc[i]])), i
 
 
-def _limit(e, members=256, join_ticks=3000, wait_polls=1 << 22):
+def _limit(e, members=256, join_ticks=3000, wait_polls=1 << 27):
     """How the workgroups of e's rebuilds meet from here on."""
     e._check(e.lib.beads_internal_rebuild_limits(e.handle, C.c_uint32(members),
                                                  C.c_int64(join_ticks), C.c_uint32(wait_polls)))
