@@ -370,6 +370,12 @@ __device__ __forceinline__ int x_bin(real_t x, real_t lo, real_t inv, uint32_t c
                         : (f >= static_cast<real_t>(kXBins - 1) ? kXBins - 1 : static_cast<int>(f));
 }
 
+// The order's key: NaN, which no comparison would place (two members would take
+// one entry and another keep what was there before), comes last.
+__device__ __forceinline__ real_t order_key(real_t x) {
+  return x == x ? x : static_cast<real_t>(__builtin_huge_val());
+}
+
 __device__ __forceinline__ bool before_in_cell(real_t xa, uint32_t sa, real_t xb, uint32_t sb) {
   return xa < xb || (xa == xb && sa < sb);
 }
@@ -385,7 +391,7 @@ __device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, b
   if (cnt <= 64) {
     const uint32_t v = lane < cnt ? agent_load(a + b + lane) : 0xffffffffu;
     const real4 xv4 = lane < cnt ? p.pos[v] : make_real4(0, 0, 0, 0);
-    const real_t xv = xv4.x;
+    const real_t xv = order_key(xv4.x);
     uint32_t rank = 0;
     for (uint32_t m = 0; m < cnt; ++m) {
       const uint32_t w = static_cast<uint32_t>(
@@ -413,9 +419,9 @@ __device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, b
     a[b] = agent_load(a + b);
     for (uint32_t k = b + 1; k < e; ++k) {
       const uint32_t v = agent_load(a + k);
-      const real_t xv = p.pos[v].x;
+      const real_t xv = order_key(p.pos[v].x);
       uint32_t m = k;
-      while (m > b && before_in_cell(xv, v, p.pos[a[m - 1]].x, a[m - 1])) {
+      while (m > b && before_in_cell(xv, v, order_key(p.pos[a[m - 1]].x), a[m - 1])) {
         a[m] = a[m - 1];
         --m;
       }
