@@ -338,8 +338,8 @@ __device__ __forceinline__ void scatter_atom(const CellScanParams& p, uint32_t i
 // scan a row as one run and skip its ends beyond r_s (cell_xbins). One wave
 // per cell: for up to 64 members lane l holds member l, whose rank is the
 // number of members before it in (x, slot) order, and stores it at start +
-// rank; the x-bin prefix counts come from one ballot per bin. A larger cell
-// is insertion-sorted by lane 0. When no reorder follows, the kernel also
+// rank; the x-bin prefix counts come from one ballot per bin. Larger cells:
+// sort_large_cell. When no reorder follows, the kernel also
 // writes the members' positions in cell order with the slot in .w (the
 // build's candidate stream); after a reorder, commit_atom writes them.
 __device__ __forceinline__ real4 cell_entry(real4 x, uint32_t slot) {
@@ -380,8 +380,71 @@ __device__ __forceinline__ bool before_in_cell(real_t xa, uint32_t sa, real_t xb
   return xa < xb || (xa == xb && sa < sb);
 }
 
-// One wave orders cell c; stream: also write the candidate stream.
-__device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, bool stream) {
+// Position of member v (x = its key) of a wave's chunk of cnt members, one a lane.
+__device__ __forceinline__ uint32_t rank_in_chunk(uint32_t v, real_t x, uint32_t cnt) {
+  uint32_t rank = 0;
+  for (uint32_t m = 0; m < cnt; ++m) {
+    const uint32_t w = static_cast<uint32_t>(
+        __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(m)));
+    const real_t xw = read_lane(x, static_cast<int>(m));
+    rank += before_in_cell(xw, w, x, v) ? 1u : 0u;
+  }
+  return rank;
+}
+
+// The members [b, b + cnt) of a cell of more than 64, ordered by one wave:
+// chunks of 64 by rank, then runs of twice the length until one is left, each
+// member's place in the other run found by bisection. The passes go back and
+// forth between cell_atoms and scratch; returns the array with the last one's
+// result. Such cells are rare, but have to end: a system that has flown apart
+// has all its atoms in the corner cells, and one lane inserting one member after
+// another took m^2 / 4 moves of 0.4 us (80 ms at 937 members, 1.5 hours at
+// 242,771, which take 155 ms now: a chain of dependent loads per bisection).
+__device__ __forceinline__ const uint32_t* sort_large_cell(const CellScanParams& p, uint32_t b,
+                                                        uint32_t cnt, uint32_t* scratch) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t *src = p.cell_atoms + b, *dst = scratch + b;
+  auto key = [&p](uint32_t v) { return order_key(p.pos[v].x); };
+  for (uint32_t base = 0; base < cnt; base += 64) {
+    const uint32_t here = min(64u, cnt - base);
+    const uint32_t v = lane < here ? agent_load(src + base + lane) : 0xffffffffu;
+    const real_t x = lane < here ? key(v) : real_t(0);
+    const uint32_t rank = rank_in_chunk(v, x, here);
+    if (lane < here) dst[base + rank] = v;
+  }
+  for (uint32_t w = 64; w < cnt; w *= 2) {  // cnt < 2^28
+    uint32_t* const done = dst;
+    dst = src;
+    src = done;
+    // The wave's stores are in the caches it reads through.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    for (uint32_t k = lane; k < cnt; k += 64) {
+      const uint32_t first = k & ~(w - 1);  // of the member's run
+      const uint32_t pair = k & ~(2 * w - 1);
+      const uint32_t other = first == pair ? first + w : pair;
+      uint32_t lo = other, hi = other < cnt ? min(cnt, other + w) : other;
+      const uint32_t v = src[k];
+      const real_t x = key(v);
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi) / 2;
+        const uint32_t u = src[mid];
+        if (before_in_cell(key(u), u, x, v)) {
+          lo = mid + 1;
+        } else {
+          hi = mid;
+        }
+      }
+      dst[pair + (k - first) + (lo - other)] = v;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  return dst - b;
+}
+
+// One wave orders cell c; stream: also write the candidate stream. scratch: an
+// entry per atom, used for large cells.
+__device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, bool stream,
+                                          uint32_t* scratch) {
   const uint32_t lane = threadIdx.x & 63u;
   const real_t lo = p.box.lo[0], inv = p.grid.inv_cell[0];
   const uint32_t b = agent_load(p.cell_start + c), e = agent_load(p.cell_start + c + 1);
@@ -392,13 +455,7 @@ __device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, b
     const uint32_t v = lane < cnt ? agent_load(a + b + lane) : 0xffffffffu;
     const real4 xv4 = lane < cnt ? p.pos[v] : make_real4(0, 0, 0, 0);
     const real_t xv = order_key(xv4.x);
-    uint32_t rank = 0;
-    for (uint32_t m = 0; m < cnt; ++m) {
-      const uint32_t w = static_cast<uint32_t>(
-          __builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(m)));
-      const real_t xw = read_lane(xv, static_cast<int>(m));
-      rank += before_in_cell(xw, w, xv, v) ? 1u : 0u;
-    }
+    const uint32_t rank = rank_in_chunk(v, xv, cnt);
     if (lane < cnt) {
       a[b + rank] = v;
       if (stream) p.cell_pos[b + rank] = cell_entry(xv4, v);
@@ -413,32 +470,27 @@ __device__ __forceinline__ void sort_cell(const CellScanParams& p, uint32_t c, b
       p.cell_xbins[c] = make_uint4(pre[0] | (pre[1] << 16), pre[2] | (pre[3] << 16),
                                    pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
     }
-  } else if (lane == 0) {
-    // Entry k as the scatter left it is another workgroup's store (agent_load);
-    // those below k are this lane's own by then.
-    a[b] = agent_load(a + b);
-    for (uint32_t k = b + 1; k < e; ++k) {
-      const uint32_t v = agent_load(a + k);
-      const real_t xv = order_key(p.pos[v].x);
-      uint32_t m = k;
-      while (m > b && before_in_cell(xv, v, order_key(p.pos[a[m - 1]].x), a[m - 1])) {
-        a[m] = a[m - 1];
-        --m;
-      }
-      a[m] = v;
-    }
-    uint32_t pre[kXBins] = {};
-    for (uint32_t k = b; k < e; ++k) {
-      const uint32_t v = a[k];
+    return;
+  }
+  const uint32_t* const sorted = sort_large_cell(p, b, cnt, scratch);
+  uint32_t pre[kXBins] = {};
+  for (uint32_t k = lane; k - lane < cnt; k += 64) {
+    int bin = kXBins;
+    if (k < cnt) {
+      const uint32_t v = sorted[b + k];
       const real4 xv4 = p.pos[v];
-      if (stream) p.cell_pos[k] = cell_entry(xv4, v);
-      const int bin = x_bin(xv4.x, lo, inv, cx);
-      for (int m = bin + 1; m <= kXBins; ++m) ++pre[m - 1];
+      a[b + k] = v;
+      if (stream) p.cell_pos[b + k] = cell_entry(xv4, v);
+      bin = x_bin(order_key(xv4.x), lo, inv, cx);
     }
-    if (cnt <= kXBinsMaxCount) {
-      p.cell_xbins[c] = make_uint4(pre[0] | (pre[1] << 16), pre[2] | (pre[3] << 16),
-                                   pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
+#pragma unroll
+    for (int m = 1; m <= kXBins; ++m) {
+      pre[m - 1] += static_cast<uint32_t>(__builtin_popcountll(__ballot(bin < m)));
     }
+  }
+  if (lane == 0 && cnt <= kXBinsMaxCount) {
+    p.cell_xbins[c] = make_uint4(pre[0] | (pre[1] << 16), pre[2] | (pre[3] << 16),
+                                 pre[4] | (pre[5] << 16), pre[6] | (pre[7] << 16));
   }
 }
 
@@ -651,7 +703,7 @@ __global__ __launch_bounds__(kRebuildBlock) void rebuild_kernel(CellScanParams c
   if (!member_barrier<false>(ctrl, m)) return;
   for (uint32_t c = m.rank * kRebuildWaves + threadIdx.x / 64; c < cp.n_cells;
        c += m.count * kRebuildWaves) {  // uniform over the wave
-    sort_cell(cp, c, !reorder);
+    sort_cell(cp, c, !reorder, rp.new_of_old);
   }
   if (!reorder) return;
   if (!member_barrier<true>(ctrl, m)) return;

@@ -34,10 +34,8 @@ struct RebuildLimits {
   int64_t join_ticks = 3000;             // how long the first waits for the grid to start,
                                          // in wall_clock64 ticks (rebuild_join_ticks)
   // Polls before any other wait is given up: at about a microsecond each some
-  // two minutes of running, far above the longest phase (one lane sorts a cell
-  // of more than 64 members, with m^2 / 4 moves of 0.4 us: 80 ms at 937 members,
-  // and so 2.3 s at 5,000; a run whose atoms have all become NaN has them in one
-  // cell, a microsecond or two each). Polls and not time, which passes for a
+  // two minutes of running, far above the longest phase (one wave orders a large
+  // cell: 155 ms at 242,771 members). Polls and not time, which passes for a
   // workgroup whose queue is off the GPU too.
   uint32_t wait_polls = 1u << 27;
 };

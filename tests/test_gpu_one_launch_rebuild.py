@@ -71,11 +71,11 @@ def test_more_cells_than_one_prefix():
     _final_state(w, 24)
 
 
-@pytest.mark.parametrize("n,steps", [(6000, 10), (30000, 48)])
-def test_cells_of_more_than_a_wave(n, steps):
-    """One lane sorts such a cell, from entries that other workgroups scattered
-    (at 30,000 beads over a hundred of them)."""
-    w = _every_step(W.lj_box(n, 0.8, 1.0, seed=4, cutoff=5.0)).with_(max_neighbors=768)
+@pytest.mark.parametrize("n,steps,cutoff", [(6000, 10, 5.0), (30000, 48, 5.0), (7000, 10, 6.0)])
+def test_cells_of_more_than_a_wave(n, steps, cutoff):
+    """One wave orders such a cell in chunks and runs of chunks, from entries that
+    other workgroups scattered (at 30,000 beads over a hundred of them)."""
+    w = _every_step(W.lj_box(n, 0.8, 1.0, seed=4, cutoff=cutoff)).with_(max_neighbors=1024)
     assert w.n / O.plan(w).n_cells > 64
     _final_state(w, steps)
 

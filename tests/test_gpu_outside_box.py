@@ -17,12 +17,12 @@ from gpu_cases import elongated_lj
 pytestmark = pytest.mark.gpu
 
 
-def _flying(w, count, seed):
+def _flying(w, count, seed, speed=4e9):
     """w with count atoms that a step carries millions of box lengths away."""
     rng = np.random.default_rng(seed)
     v = w.velocities.copy()
     fast = rng.choice(w.n, size=count, replace=False)
-    v[fast] = (rng.standard_normal((count, 3)) * 4e9).astype(np.float32)
+    v[fast] = (rng.standard_normal((count, 3)) * speed).astype(np.float32)
     return w.with_(velocities=v, cutoff_buffer=0.0, max_neighbors=256)
 
 
@@ -58,3 +58,19 @@ def test_lists_are_the_full_scans(make, count, half):
     np.testing.assert_array_equal(counts, (want != 0xffffffff).sum(axis=1))
     assert np.array_equal(np.sort(got, axis=0).T, np.sort(want, axis=1))
 
+
+def test_all_atoms_in_the_corner_cells():
+    """Farther still, and the wrap leaves every atom far outside: the corner
+    cells hold them all, and their members come in order of x."""
+    w = _flying(W.lj_box(40000, 0.8, 1.0, seed=7), 40000, seed=7, speed=4e12)
+    plan = O.plan(w)
+    with Engine(w) as e:
+        e.initialize(observables=False)
+        e.advance(1)
+        st, cells = e.state(), e.cells(plan.n_cells)
+    ref = O.cell_ids(w, positions=st["positions"])
+    order, counts, offsets = O.stable_cell_order(ref, plan.n_cells, st["positions"])
+    assert counts.max() > 2000
+    np.testing.assert_array_equal(cells["cell_count"], counts)
+    np.testing.assert_array_equal(cells["cell_start"], offsets)
+    np.testing.assert_array_equal(cells["cell_atoms"], order)
